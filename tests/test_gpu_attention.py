@@ -706,3 +706,40 @@ def test_small_prefill_batches_split_their_keys_and_match_the_oracle(case):
             _lib.ATTN_NO_DECODE_ROWS, None, 0, stream_handle()))
         assert max_abs(plain, want) <= tol
         assert max_abs(plain, got) <= tol
+
+
+# ---- the order of a prefill launch's work items -------------------------------
+
+ORDER_CASES = [
+    # dtype, heads, kvh, d, n_seqs: tiles of 256 rows (128 at head_dim 256)
+    (torch.bfloat16, 4, 1, 64, 2),     # two sequences: the smallest sorted list
+    (torch.float16, 21, 3, 128, 9),    # kv heads that do not divide the XCDs
+    (torch.bfloat16, 32, 8, 128, 64),  # one sequence per lane
+    (torch.bfloat16, 16, 2, 64, 65),   # past the sort: list order
+    (torch.bfloat16, 8, 2, 256, 5),
+]
+
+
+@pytest.mark.parametrize("case", ORDER_CASES, ids=lambda c: f"{str(c[0])[6:]}-kvh{c[2]}-d{c[3]}-n{c[4]}")
+def test_every_tile_of_a_ragged_prefill_batch_is_computed_once(case):
+    """Prefill batches of very different lengths (one tile beside several,
+    equal contexts, decode rows between them when a list names the prefill
+    ones) match the oracle whatever order the launch walks the tiles in."""
+    dtype, heads, kvh, d, n = case
+    rng = np.random.default_rng(zlib.crc32(str(case).encode()))
+    rows = 128 if d == 256 else 256
+    tile = rows * kvh // heads  # query tokens per tile
+    lens_q = [int(x) for x in rng.integers(2, tile + 3, n)]
+    lens_q[0], lens_q[-1] = 2 * tile + 1, tile
+    lens_k = [l + int(x) for l, x in zip(lens_q, rng.integers(0, 40, n))]
+    lens_k[-1] = max(lens_k[0], lens_q[-1])  # equal contexts: a tie in the order
+    for decode_rows in (False, True):
+        if decode_rows:
+            lens_q[n // 2] = 1
+        c, q, batch = random_case(rng, dtype, heads, kvh, d, 16, lens_q, lens_k, "HND")
+        prep = PreparedAttention.from_batch(batch, DEV, cache=c, num_heads=heads)
+        want = oracle_out(q, c, 0, batch, d ** -0.5)
+        got = torch.full_like(q, float("nan"))
+        paged_attention_prepared(q, c, 0, prep, d ** -0.5, out=got)
+        tol = (2e-2 if dtype == torch.bfloat16 else 1e-2) * float(want.abs().max())
+        assert max_abs(got, want) <= tol

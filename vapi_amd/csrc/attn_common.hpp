@@ -70,6 +70,7 @@ struct AttnArgs {
   // batch - 1); the host names the sequences with prefill rows.
   const uint32_t* pf_seqs;
   uint32_t pf_seqs_n;
+  uint32_t pf_sort;  // prefill: items in descending order of work (prefill_sorts)
   // decode: a group of G > 16 query heads per kv head runs as n = kv_parts
   // virtual kv heads of P = group = ceil(G / n) query heads each (kvh and
   // group then count the virtual ones; the last part of a group may hold
@@ -99,6 +100,90 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t lin, uint32_t n) {
   const uint32_t x = lin % kXcds, i = lin / kXcds;
   const uint32_t per = n / kXcds, extra = n % kXcds;  // XCD x gets per + (x < extra)
   return x * per + min(x, extra) + i;
+}
+
+// A prefill work item: query tile qt of list entry li (sequence seq, its rows
+// q0 .. q0 + len_q - 1 and context len_k), kv head kh.
+struct PfItem {
+  uint32_t li, seq, qt, kh, q0, len_q;
+  int32_t len_k;
+};
+
+// Item `i` of a prefill launch over a.pf_seqs_n list entries of at most
+// `qtiles` tiles of `rows` rows each; false when there is none (a sequence
+// with fewer tiles than the longest leaves items over). The kv head is the
+// fastest index, so the hardware's round-robin dealing over the 8 XCDs gives
+// every XCD the same tiles of its own heads (with 8 kv heads, one head each:
+// the tiles of a sequence that run together share K/V under one L2), and
+// the heads' equal work balances the XCDs whatever the lengths are. Up to
+// kPfSortSeqs sequences are walked from the longest context to the shortest
+// and each from its last tile to its first (the causal mask makes later
+// tiles longer), so the last items handed out are short; empty items all
+// come last. Against contiguous item ranges per XCD in list order: seven
+// fresh f16 prompts of 40-2,943 tokens (28 q / 4 kv heads) 404 -> 181 us
+// (the longest prompt's tiles had all run on one XCD), 16 chunks of 30-1,500
+// over ~500 earlier keys (32 q / 32 kv heads) 484 -> 295 us, config 3's
+// equal sequences 1,065 -> 1,057 us. Launches of one tile per sequence and
+// of more sequences than lanes keep list order, which needs no walk over
+// the list (64 sequences of 32 fresh tokens: 16.8 us, 18.2 sorted; 17.4
+// before).
+// Each of the workgroup's W waves holds one sequence per lane and counts the
+// tiles before it among its share of the others; `tmp` (W x 64 words of LDS)
+// adds the shares up. Every thread of the workgroup calls this.
+constexpr uint32_t kPfSortSeqs = 64;
+inline bool prefill_sorts(uint32_t n_seqs, uint32_t qtiles) {
+  return n_seqs > 1 && n_seqs <= kPfSortSeqs && qtiles > 1;
+}
+template <int W>
+__device__ __forceinline__ bool prefill_item(const AttnArgs& a, const uint32_t* __restrict__ cu_q,
+                                             const uint32_t* __restrict__ cu_k, uint32_t i,
+                                             uint32_t qtiles, uint32_t rows, uint32_t* tmp,
+                                             PfItem& it) {
+  const uint32_t rank = i / a.kvh, n = a.pf_seqs_n;
+  it.kh = i - rank * a.kvh;
+  if (!a.pf_sort) {
+    it.li = rank / qtiles;
+    it.qt = qtiles - 1 - (rank - it.li * qtiles);
+    it.seq = a.pf_seqs ? a.pf_seqs[it.li] : it.li;
+    if (it.seq >= a.batch) return false;
+    it.q0 = cu_q[it.seq];
+    it.len_q = cu_q[it.seq + 1] - it.q0;
+    it.len_k = (int32_t)(cu_k[it.seq + 1] - cu_k[it.seq]);
+    return it.len_q >= a.pf_min_q && it.len_q > 0;
+  }
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t seq = 0, nt = 0, key = 0, q0 = 0, len_q = 0;
+  if (lane < n) {
+    seq = a.pf_seqs ? a.pf_seqs[lane] : lane;
+    if (seq < a.batch) {
+      q0 = cu_q[seq], len_q = cu_q[seq + 1] - q0;
+      key = cu_k[seq + 1] - cu_k[seq];
+      if (len_q >= a.pf_min_q && len_q > 0)
+        nt = min((uint32_t)(((uint64_t)len_q * a.group + rows - 1) / rows), qtiles);
+    }
+  }
+  // Tiles of the sequences walked before this lane's.
+  uint32_t start = 0;
+  for (uint32_t s = wave; s < n; s += W) {
+    const uint32_t ks = __builtin_amdgcn_readlane(key, s), ns = __builtin_amdgcn_readlane(nt, s);
+    start += ks > key || (ks == key && s < lane) ? ns : 0u;
+  }
+  tmp[wave * 64 + lane] = start;
+  __syncthreads();
+  start = 0;
+#pragma unroll
+  for (int w = 0; w < W; ++w) start += tmp[w * 64 + lane];
+  const uint64_t hit = __ballot(rank >= start && rank - start < nt);
+  if (hit == 0) return false;
+  it.li = (uint32_t)__builtin_ctzll(hit);
+  it.seq = __builtin_amdgcn_readlane(seq, it.li);
+  it.qt = __builtin_amdgcn_readlane(nt, it.li) - 1 -
+          (rank - __builtin_amdgcn_readlane(start, it.li));
+  it.q0 = __builtin_amdgcn_readlane(q0, it.li);
+  it.len_q = __builtin_amdgcn_readlane(len_q, it.li);
+  it.len_k = (int32_t)__builtin_amdgcn_readlane(key, it.li);
+  return true;
 }
 
 // ---------------------------------------------------------------------------

@@ -169,7 +169,7 @@ __device__ __forceinline__ void lgkm_wait(uint2 (&r)[4]) {
 // contiguous runs of steps, one workgroup each (a batch too small to fill
 // the GPU with query tiles alone); each writes its rows' (m, l, o) to
 // `part` and paged_prefill_merge combines them.
-// Workgroup `bid` of `n_items` (W waves) of a prefill launch.
+// Workgroup `bid` (W waves) of a prefill launch.
 // DL: the 16-column d tiles that hold head_dim (kPad; D / 16 otherwise):
 // the score MFMAs, V^T reads, PV MFMAs and stores of the tiles past them
 // are left out.
@@ -177,7 +177,7 @@ template <typename T, int D, int RT, int W, bool kSplit, bool kPad = false, int 
 __device__ __forceinline__ void prefill_body(
     const AttnArgs& a, const uint32_t* __restrict__ cu_q, const uint32_t* __restrict__ cu_k,
     const uint32_t* __restrict__ table, uint32_t qtiles, uint32_t n_split_arg,
-    float* __restrict__ part, uint32_t bid, uint32_t n_items) {
+    float* __restrict__ part, uint32_t bid) {
   // The unsplit launch compiles without the split's arithmetic.
   const uint32_t n_split = kSplit ? n_split_arg : 1u;
   static_assert(W == 8 || W == 4, "a step's K and V are loaded by 8 or 4 waves");
@@ -196,17 +196,16 @@ __device__ __forceinline__ void prefill_body(
   // every LDS read.
   __shared__ __attribute__((aligned(16))) uint16_t k0[32 * D], k1[32 * D], k2[32 * D];
   __shared__ __attribute__((aligned(16))) uint16_t v0[32 * D], v1[32 * D], v2[32 * D];
-  const uint32_t item = xcd_remap(bid, n_items);
-  // Item order: query tile fastest, then key split, kv head, sequence (the
-  // q-tiles of one split read the same K/V and run on one XCD).
-  const uint32_t qt = item % qtiles, rest_s = item / qtiles;
-  const uint32_t split = rest_s % n_split, rest = rest_s / n_split;
-  const uint32_t kh = rest % a.kvh;
-  const uint32_t seq = a.pf_seqs ? a.pf_seqs[rest / a.kvh] : rest / a.kvh;
-  if (seq >= a.batch) return;
-  const uint32_t q0 = cu_q[seq];
-  const uint32_t len_q = cu_q[seq + 1] - q0;
-  if (len_q < a.pf_min_q || len_q == 0) return;
+  // Item order: kv head fastest, then key split, then query tile (the split
+  // index counts per tile, so the items of one tile stay together).
+  __shared__ uint32_t order[64 * W];
+  const uint32_t hr = bid / a.kvh, split = hr % n_split;
+  PfItem it;
+  if (!prefill_item<W>(a, cu_q, cu_k, (hr / n_split) * a.kvh + bid % a.kvh, qtiles, kPfRows,
+                       order, it))
+    return;
+  const uint32_t qt = it.qt, kh = it.kh, seq = it.seq, rest = it.li * a.kvh + kh;
+  const uint32_t q0 = it.q0, len_q = it.len_q;
   const uint32_t G = a.group;
   const uint32_t nrows = len_q * G;
   const uint32_t row_base = qt * kPfRows;
@@ -214,7 +213,7 @@ __device__ __forceinline__ void prefill_body(
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t col = lane & 15, g = lane >> 4;
-  const int32_t len_k = (int32_t)(cu_k[seq + 1] - cu_k[seq]);
+  const int32_t len_k = it.len_k;
   const int32_t offset = len_k - (int32_t)len_q;
   const int32_t last = len_k - 1;
 
@@ -452,7 +451,7 @@ __global__ __launch_bounds__(kPfThreads, OCC) void paged_prefill_tiled(
     const uint32_t* __restrict__ table, uint32_t qtiles, uint32_t n_split_arg,
     float* __restrict__ part) {
   prefill_body<T, D, RT, kPfWaves, kSplit, kPad, DL>(a, cu_q, cu_k, table, qtiles, n_split_arg, part,
-                                           blockIdx.x, gridDim.x);
+                                           blockIdx.x);
 }
 
 // Combines the key splits' partials of a prefill launch: thread (row, four
@@ -611,8 +610,7 @@ __global__ __launch_bounds__(256, 2) void paged_mixed_stream(AttnArgs a, uint32_
     decode_stream_body<T, D, false, kPad>(a, a.cu_q, a.cu_k, a.table, P, blockIdx.x, nwg);
   else {
     prefill_body<T, D, kMixRowTiles, kMixPfWaves, kSplit, kPad>(a, a.cu_q, a.cu_k, a.table, qtiles,
-                                                          n_split, part, blockIdx.x - nwg,
-                                                          gridDim.x - nwg);
+                                                          n_split, part, blockIdx.x - nwg);
   }
 }
 
@@ -640,6 +638,7 @@ void launch_mixed(const AttnArgs& a_in, void* workspace, uint32_t max_q, uint32_
   decode_bind(c, workspace, head_dim);
   const uint32_t nwg = c.num_waves / kDecodeWavesPerWG;
   const uint32_t qtiles = (uint32_t)(((uint64_t)max_q * c.group + kMixRows - 1) / kMixRows);
+  c.pf_sort = prefill_sorts(c.pf_seqs_n, qtiles);
   const uint64_t base = (uint64_t)qtiles * c.kvh * c.pf_seqs_n;
   // The prefill workgroups run beside the decode's, one per CU: as many key
   // splits as keep them within one round of the GPU's CUs (a second round
@@ -726,6 +725,7 @@ void launch_prefill(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, uint32
   AttnArgs a = a_in;
   const uint32_t rows = pf_rows(head_dim);
   const uint32_t qtiles = (uint32_t)(((uint64_t)max_q * a.group + rows - 1) / rows);
+  a.pf_sort = prefill_sorts(a.pf_seqs_n, qtiles);
   const uint64_t base = (uint64_t)qtiles * a.kvh * a.pf_seqs_n;
   // As many splits as the workspace given holds (none without one); a
   // deterministic call does not split, so its output does not depend on
