@@ -743,3 +743,72 @@ def test_every_tile_of_a_ragged_prefill_batch_is_computed_once(case):
         paged_attention_prepared(q, c, 0, prep, d ** -0.5, out=got)
         tol = (2e-2 if dtype == torch.bfloat16 else 1e-2) * float(want.abs().max())
         assert max_abs(got, want) <= tol
+
+
+# ---- f32 prefill by three-way bf16 splits -------------------------------------
+
+X3_CASES = [
+    # heads, kvh, d, bs, lens_q, lens_k, window, layout: items of 128 rows
+    (8, 4, 128, 16, [2], [33], None, "HND"),           # the smallest, few kv heads
+    (16, 8, 128, 16, [64, 63, 65], [64, 95, 300], None, "HND"),  # a full tile and its edges
+    (28, 4, 64, 32, [40, 130], [700, 1100], 257, "NHD"),
+    (16, 4, 20, 16, [50], [90], None, "HND"),          # one live chunk of head_dim 64's
+    (8, 2, 72, 16, [100, 33], [161, 33], 64, "HND"),   # half of a 16-column tile
+    (8, 8, 96, 16, [300], [777], None, "NHD"),
+    (8, 8, 116, 16, [130, 2], [200, 2], None, "HND"),  # an odd half chunk
+    (64, 8, 128, 16, [1100], [1100], None, "HND"),     # enough items for two row tiles per wave
+    (64, 8, 60, 16, [1040], [1100], 333, "HND"),
+]
+
+
+@pytest.mark.parametrize("case", X3_CASES, ids=lambda c: f"g{c[0] // c[1]}-d{c[2]}-q{c[4]}-w{c[6]}")
+def test_f32_prefill_by_bf16_splits_matches_within_1e_5(case):
+    """Against the oracle at the f32 bar, without a workspace too."""
+    heads, kvh, d, bs, lens_q, lens_k, window, layout = case
+    rng = np.random.default_rng(zlib.crc32(str(case).encode()))
+    c, q, batch = random_case(rng, torch.float32, heads, kvh, d, bs, lens_q, lens_k, layout)
+    want = oracle_out(q, c, 0, batch, d ** -0.5, window)
+    for det in (False, True):  # deterministic: no key split
+        prep = PreparedAttention.from_batch(batch, DEV, cache=c, num_heads=heads,
+                                            deterministic=det)
+        got = torch.full_like(q, float("nan"))
+        paged_attention_prepared(q, c, 0, prep, d ** -0.5, None if window is None else window - 1,
+                                 out=got)
+        assert max_abs(got, want) <= 1e-5
+
+
+@pytest.mark.parametrize("what", ["k_inf", "v_max", "v_tiny", "q_max", "zeros"])
+@pytest.mark.parametrize("det", [False, True])
+def test_f32_prefill_of_values_without_a_bf16_split(what, det):
+    """Infinities, values above the largest bf16 and tensors of tiny values
+    take the f32 MFMAs inside the same launch, split or not."""
+    rng = np.random.default_rng(3)
+    c, q, batch = random_case(rng, torch.float32, 8, 4, 128, 16, [70, 40], [600, 90], "HND")
+    big = float(np.finfo(np.float32).max)
+    unit = 1.0
+    if what == "k_inf":  # scores of -inf for one key per block
+        q[..., 0] = q[..., 0].abs() + 0.1
+        c.k[0][:, :, 3, 0] = -float("inf")
+    elif what == "v_max":
+        # One key of the first tile, which sets the running max: the online
+        # softmax's unnormalised weight of a later key may exceed 1 and take
+        # the sum past the largest float.
+        c.v[0][batch.block_tables[0][0], :, 5, 7] = big
+        unit = big
+    elif what == "v_tiny":
+        unit = 2.0 ** -118
+        c.v[0].mul_(unit)
+    elif what == "q_max":
+        q.mul_(1e-30)
+        q[:, :, 1] = big
+        c.k[0].mul_(1e-38)
+    else:
+        c.k[0].zero_()
+        c.v[0].zero_()
+    want = oracle_out(q, c, 0, batch, 128 ** -0.5)
+    prep = PreparedAttention.from_batch(batch, DEV, cache=c, num_heads=8, deterministic=det)
+    got = torch.full_like(q, float("nan"))
+    paged_attention_prepared(q, c, 0, prep, 128 ** -0.5, out=got)
+    assert bool(torch.isfinite(want).all())
+    err = ((got.double().cpu() - want.double()) / unit).abs()
+    assert float(err.max()) <= 1e-5

@@ -5,8 +5,9 @@
 // when the pool is bf16/f16 with head_dim 64, 128 or 256, a power-of-two
 // block_size >= 16 and at most 16 query heads per kv head (up to 64 when a
 // split into 2 or 4 equal groups of at most 16 exists); an f32 pool of
-// that shape (head_dim 64 or 128) runs the decode stream and an f32 prefill
-// kernel (attn_prefill_f32.hip) on f32 MFMAs; a 16-bit decode-only call at a
+// that shape (head_dim 64 or 128) runs the decode stream on f32 MFMAs and the
+// f32 prefill kernels (attn_prefill_f32.hip: exact bf16 splits, or f32 MFMAs
+// for few rows); a 16-bit decode-only call at a
 // head_dim that is another multiple of 8 up to 256 runs the decode stream
 // padded to the next of 64, 128, 256; every other shape runs the VALU kernel
 // (attn_generic.hip).
@@ -28,8 +29,8 @@ static uint32_t decode_group_parts(uint32_t G) {
   return n <= 16 ? n : 0;
 }
 
-// An f32 pool whose calls run on v_mfma_f32_16x16x4_f32: decode rows on the
-// decode stream, prefill rows on paged_prefill_f32. A small pure-decode call
+// An f32 pool whose calls run on MFMAs: decode rows on the decode stream,
+// prefill rows on the f32 prefill kernels. A small pure-decode call
 // (at most 512 keys per sequence and 8,192 over the batch, config 0's shape)
 // runs the VALU kernel instead, in one launch with no merge. Replayed from
 // a graph, 16 q / 8 kv heads: config 0 (8 x <= 512 keys) 14.1 against

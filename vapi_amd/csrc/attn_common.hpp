@@ -729,10 +729,10 @@ uint32_t decode_max_plan_seqs();
 // Workspace the prefill's key split wants for this shape (0: no split).
 size_t prefill_split_bytes(uint32_t batch, uint32_t kvh, uint32_t group, uint32_t head_dim,
                            uint32_t max_q, uint32_t max_k);
-// Prefill rows of an f32 pool (head_dim 64 or 128) on f32 MFMAs, over
-// a.pf_seqs_n sequences; waves of the launch (a launch needs it below 2^32).
+// Prefill rows of an f32 pool (head_dim 64 or 128) over a.pf_seqs_n
+// sequences; items of the launch (a launch needs it below 2^32).
 uint64_t prefill_f32_items(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_q);
-// With a workspace (`split_ws`), a batch of fewer waves than the GPU holds
+// With a workspace (`split_ws`), a batch of fewer items than the GPU holds
 // splits its keys; the merge runs as a second launch.
 void launch_prefill_f32(const AttnArgs& a, uint32_t max_q, uint32_t max_k, uint32_t head_dim,
                         void* split_ws, size_t split_ws_bytes, hipStream_t s);
