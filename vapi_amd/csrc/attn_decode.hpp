@@ -28,7 +28,7 @@
 // launch has at most 256 segments (each then split into many pieces), one
 // workgroup per segment whose waves share its pieces. Each
 // segment's first and last range are recorded by the waves holding its first
-// and last step, and a wave whose slice is empty marks its slot empty, so
+// and last step, and every range between them holds steps of the segment, so
 // the merge needs no step arithmetic. The merge
 // kernel's extra workgroup turns the stream's per-wave timings into the
 // next launch's shares. (Merging inside the stream, by the wave that
@@ -71,16 +71,10 @@ __device__ __forceinline__ uint32_t decode_steps(const AttnArgs& a,
   return (uint32_t)(len_k - (lo & ~31) + 31) >> 5;
 }
 
-// Waves in group x and the number of waves in groups before it.
+// Waves in group x.
 __device__ __forceinline__ uint32_t group_waves(uint32_t nwg, uint32_t x) {
   return nwg > x ? ((nwg - 1 - x) / kGroups + 1) * kDecodeWavesPerWG : 0u;
 }
-__device__ __forceinline__ uint32_t group_offset(uint32_t nwg, uint32_t x) {
-  uint32_t off = 0;
-  for (uint32_t y = 0; y < x; ++y) off += group_waves(nwg, y);
-  return off;
-}
-
 // The shares of this launch: 8 positive f32, uniform when the workspace
 // holds none yet (all zero) or anything unusable; 0 for groups without waves.
 __device__ __forceinline__ void load_shares(const AttnArgs& a, uint32_t nwg, float (&w)[kGroups]) {
@@ -374,30 +368,28 @@ __device__ __forceinline__ void decode_stream_body(const AttnArgs& a,
   const uint32_t j = (bid / kGroups) * kDecodeWavesPerWG + wave;
   const uint32_t len = F[x + 1] - F[x], nw = group_waves(nwg, x);
   // The group's waves form ranges of n consecutive waves, wave j taking
-  // part j % n of range j / n (waves past the last whole range idle), so
-  // the parts of a pool head's steps are read at once, by neighbouring
-  // waves of one XCD. A piece's partial slot is r n + (virtual segment):
-  // r + (pool segment) is distinct for every piece of one part, as in the
-  // unsplit order, so the slots of all parts are too.
-  const uint32_t nr = nw / n_parts;
+  // part j % n of range j / n, so that the parts of a pool head's steps are
+  // read at once by neighbouring waves of one XCD. A group of fewer steps
+  // than ranges uses one range per step (the other waves idle), and ranges
+  // are numbered over the used ones of all groups. A piece's partial slot
+  // is r n + (virtual segment): r + (pool segment) is distinct for every
+  // piece of one part, as in the unsplit order, so the slots of all parts
+  // are too.
+  const uint32_t nr = min(nw / n_parts, len);
   const uint32_t jr = j / n_parts;
   const uint32_t part = j - jr * n_parts;
-  const uint32_t t_begin = jr < nr ? F[x] + (uint32_t)(((uint64_t)jr * len) / nr) : S;
-  const uint32_t t_end = jr < nr ? F[x] + (uint32_t)(((uint64_t)(jr + 1) * len) / nr) : S;
-  const uint32_t r = group_offset(nwg, x) / n_parts + jr;
+  uint32_t r = jr;
+#pragma unroll
+  for (uint32_t y = 0; y + 1 < kGroups; ++y)
+    r += y < x ? min(group_waves(nwg, y) / n_parts, F[y + 1] - F[y]) : 0u;
   const uint32_t gw = bid * kDecodeWavesPerWG + wave;
   uint32_t* stat = a.bal + kBalStats + kStatWords * gw;
-  if (t_begin >= t_end) {
+  if (jr >= nr) {
     if (lane == 0) *(uint4*)stat = make_uint4(0u, t_entry, t_entry, 0u);
-    // An empty slice between the first and last range of a segment: its
-    // partial slot is marked empty (l = 0) for the merge.
-    if (t_begin < S) {
-      const DecodePos p = locate(a, cu_q, cu_k, P, FZ, t_begin, kvh_plan, n_parts, part);
-      const uint64_t slot = (uint64_t)r * n_parts + p.seq * a.kvh + p.kh;
-      if (lane < a.group) *(float2*)(a.ws_ml + (slot * a.group + lane) * 2) = make_float2(kNegBig, 0.f);
-    }
     return;
   }
+  const uint32_t t_begin = F[x] + (uint32_t)(((uint64_t)jr * len) / nr);
+  const uint32_t t_end = F[x] + (uint32_t)(((uint64_t)(jr + 1) * len) / nr);
 
   uint32_t t = t_begin;
   const uint32_t col = lane & 15, g = lane >> 4;
@@ -597,7 +589,7 @@ __device__ __forceinline__ void update_shares(const AttnArgs& a, uint32_t nwg, u
 // One wave per (sequence, kv head) segment combines the segment's partials
 // if it was split; the extra last wave updates the shares. Lane l owns the
 // E = G*D/64 contiguous outputs from l*E (at most two heads), merged 8 at a
-// time over batches of 8 ranges. A partial with l = 0 is an empty slice's.
+// time over batches of 8 ranges.
 // Fused append: workgroups past the merge's write the new K/V rows to their
 // slots (the stream read them from the new rows, so no read of this launch
 // pair depends on these writes). Rows are D contiguous elements; 16-byte
@@ -727,7 +719,7 @@ __device__ __forceinline__ void decode_merge_body(const AttnArgs& a, uint32_t nw
   // segment, 8 ranges per wave measured 0.6-2.4 us faster per call than 16
   // at B = 1-16, and 4 slower at B = 1.)
   constexpr int R = 8;
-  __shared__ float cmb[WPS > 1 ? WPS : 1][3][WPS > 1 ? 64 * 8 : 1];
+  __shared__ float cmb_ml[WPS][2][2][WPS > 1 ? 64 : 1], cmb_o[WPS][8][WPS > 1 ? 64 : 1];
   for (uint32_t j0 = 0; j0 < E; j0 += 8) {
     const uint32_t n = min(8u, E - j0);
     // Running max and sum per head (a lane's eight outputs span at most two
@@ -753,7 +745,7 @@ __device__ __forceinline__ void decode_merge_body(const AttnArgs& a, uint32_t nw
         }
         const float2 x0 = in ? *(const float2*)(a.ws_ml + (sl + h0) * 2) : make_float2(kNegBig, 0.f);
         const float2 x1 = in ? *(const float2*)(a.ws_ml + (sl + h1) * 2) : make_float2(kNegBig, 0.f);
-        // Empty partials (l = 0) weigh nothing, whatever their m and o hold.
+        // Partials with l = 0 weigh nothing, whatever their m and o hold.
         mm[u][0] = x0.y > 0.f ? x0.x : kNegBig, ll[u][0] = x0.y;
         mm[u][1] = x1.y > 0.f ? x1.x : kNegBig, ll[u][1] = x1.y;
       }
@@ -778,48 +770,44 @@ __device__ __forceinline__ void decode_merge_body(const AttnArgs& a, uint32_t nw
         float Oj = O[j] * f[hw];
 #pragma unroll
         for (int u = 0; u < R; ++u) {
-          // A zero weight takes nothing from the piece's o (an empty slice's
-          // slot holds whatever an earlier call left there).
+          // A zero weight takes nothing (ranges past r1 in the batch).
           Oj += e[u][hw] != 0.f ? om[u][j] * e[u][hw] : 0.f;
         }
         O[j] = Oj;
       }
     }
-    float M[8], L[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int hw = e_lane + j0 + j >= (h0 + 1) * D;
-      M[j] = Mh[hw], L[j] = Lh[hw];
-    }
     if constexpr (WPS > 1) {
-      // The segment's waves hand their (M, L, O) to wave 0 through LDS, in
-      // wave order, so the combination order is fixed.
+      // The segment's waves exchange (M, L) per head and O through LDS, each
+      // then combining 8 / WPS of the lane's outputs over the waves in wave
+      // order (a fixed order). Lanes are the fastest index: no bank conflicts.
+      constexpr int PJ = 8 / WPS;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        cmb[v][0][lane * 8 + j] = M[j];
-        cmb[v][1][lane * 8 + j] = L[j];
-        cmb[v][2][lane * 8 + j] = O[j];
-      }
+      for (int h = 0; h < 2; ++h) cmb_ml[v][h][0][lane] = Mh[h], cmb_ml[v][h][1][lane] = Lh[h];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) cmb_o[v][j][lane] = O[j];
       __syncthreads();
-      if (v == 0) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          float Mn = M[j];
+      for (int jj = 0; jj < PJ; ++jj) {
+        const uint32_t j = v * PJ + jj;
+        const int hw = e_lane + j0 + j >= (h0 + 1) * D;
+        float m[WPS], Mn = kNegBig, Lj = 0.f, Oj = 0.f;
 #pragma unroll
-          for (int x = 1; x < WPS; ++x) Mn = fmaxf(Mn, cmb[x][0][lane * 8 + j]);
-          float Lj = 0.f, Oj = 0.f;
+        for (int x = 0; x < WPS; ++x) m[x] = cmb_ml[x][hw][0][lane], Mn = fmaxf(Mn, m[x]);
 #pragma unroll
-          for (int x = 0; x < WPS; ++x) {
-            const float f = fast_exp2(cmb[x][0][lane * 8 + j] - Mn);
-            Lj += cmb[x][1][lane * 8 + j] * f;
-            Oj += cmb[x][2][lane * 8 + j] * f;
-          }
-          L[j] = Lj, O[j] = Oj;
+        for (int x = 0; x < WPS; ++x) {
+          const float f = fast_exp2(m[x] - Mn);
+          Lj += cmb_ml[x][hw][1][lane] * f;
+          Oj += cmb_o[x][j][lane] * f;
         }
-        store(e_lane + j0, n, O, L);
+        const uint32_t e = e_lane + j0 + j;
+        if (j < n && e < e_end && (!kPad || e % D < hd))
+          orow[kPad ? (e / D) * hd + e % D : e] = from_f32<T>(Lj > 0.f ? Oj / Lj : 0.f);
       }
-      __syncthreads();  // cmb is reused by the next eight outputs
+      __syncthreads();  // the LDS is reused by the next eight outputs
     } else {
+      float L[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) L[j] = Lh[e_lane + j0 + j >= (h0 + 1) * D];
       store(e_lane + j0, n, O, L);
     }
   }
