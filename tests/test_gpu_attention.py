@@ -812,3 +812,56 @@ def test_f32_prefill_of_values_without_a_bf16_split(what, det):
     assert bool(torch.isfinite(want).all())
     err = ((got.double().cpu() - want.double()) / unit).abs()
     assert float(err.max()) <= 1e-5
+
+
+# ---- short decodes: a workgroup (or a few) per sequence and kv head -----------
+
+SMALL_CASES = [
+    # dtype, heads, kvh, d, bs, lens_k, window, layout
+    (torch.bfloat16, 4, 1, 128, 16, [1, 31, 32, 33, 256, 257], None, "HND"),
+    (torch.bfloat16, 32, 8, 128, 16, [480] * 32, None, "NHD"),   # 256 workgroups, unsplit
+    (torch.bfloat16, 32, 8, 128, 16, [479, 1, 300], None, "HND"),  # under the split's line
+    (torch.bfloat16, 32, 8, 128, 16, [481, 2, 95], None, "HND"),   # over it: empty shares
+    (torch.float16, 28, 4, 128, 32, [5000, 40], None, "HND"),      # 32 shares
+    (torch.bfloat16, 16, 16, 96, 16, [900, 640, 33], 257, "NHD"),  # padded, windowed
+    (torch.float16, 26, 2, 64, 16, [700, 900], 33, "HND"),         # 13 query heads
+    (torch.bfloat16, 14, 2, 256, 16, [300, 900], None, "HND"),
+    (torch.bfloat16, 10, 2, 200, 16, [50, 230], None, "HND"),
+    (torch.float32, 16, 8, 128, 16, [64, 95, 97, 512], None, "HND"),
+    (torch.float32, 6, 2, 36, 16, [700, 12], 100, "NHD"),
+    (torch.float32, 24, 2, 64, 64, [1500], None, "HND"),           # past the VALU kernel's sizes
+]
+
+
+@pytest.mark.parametrize("case", SMALL_CASES,
+                         ids=lambda c: f"{str(c[0])[6:]}-g{c[1] // c[2]}-d{c[3]}-n{len(c[5])}-w{c[6]}")
+def test_short_decodes_match_the_oracle(case):
+    """With and without a workspace for partials beyond the call's need, and
+    bit for bit the same on a second call."""
+    dtype, heads, kvh, d, bs, lens_k, window, layout = case
+    rng = np.random.default_rng(zlib.crc32(str(case).encode()))
+    c, q, batch = random_case(rng, dtype, heads, kvh, d, bs, [1] * len(lens_k), lens_k, layout)
+    want = oracle_out(q, c, 0, batch, d ** -0.5, window)
+    tol = (1e-5 if dtype == torch.float32 else
+           (2e-2 if dtype == torch.bfloat16 else 1e-2) * float(want.abs().max()))
+    prep = PreparedAttention.from_batch(batch, DEV, cache=c, num_heads=heads)
+    got = torch.full_like(q, float("nan"))
+    left = None if window is None else window - 1
+    paged_attention_prepared(q, c, 0, prep, d ** -0.5, left, out=got)
+    assert max_abs(got, want) <= tol
+    assert torch.equal(paged_attention_prepared(q, c, 0, prep, d ** -0.5, left), got)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_keys_outside_a_short_decodes_range_do_not_reach_its_output(dtype):
+    """Infinities in the pool's rows past the sequence's last key and before
+    its window's first one leave the output as it is without them."""
+    rng = np.random.default_rng(9)
+    c, q, batch = random_case(rng, dtype, 8, 2, 128, 16, [1, 1], [150, 39], "HND")
+    prep = PreparedAttention.from_batch(batch, DEV, cache=c, num_heads=8)
+    want = paged_attention_prepared(q, c, 0, prep, 128 ** -0.5, 20)
+    for t, n in zip(batch.block_tables, (150, 39)):
+        for pos in list(range(max(n - 1 - 20 - 31, 0), n - 1 - 20)) + list(range(n, len(t) * 16)):
+            c.k[0][t[pos // 16], :, pos % 16] = float("inf")
+            c.v[0][t[pos // 16], :, pos % 16] = -float("inf")
+    assert torch.equal(paged_attention_prepared(q, c, 0, prep, 128 ** -0.5, 20), want)

@@ -37,13 +37,15 @@ COMMON_FLAGS = [
     f"-I{ROOT / 'include'}",
 ]
 
-SOURCES = ["kv_ops.hip", "attention.hip", "attn_decode.hip", "attn_prefill.hip",
-           "attn_prefill_f32.hip", "attn_generic.hip", "host.cpp", "spill.cpp"]
+SOURCES = ["kv_ops.hip", "attention.hip", "attn_decode.hip", "attn_decode_small.hip",
+           "attn_prefill.hip", "attn_prefill_f32.hip", "attn_generic.hip", "host.cpp", "spill.cpp"]
 
 # The MFMA attention kernels never produce NaN from finite K/V/Q (masked
 # scores are -inf, running maxima start finite), so fmaxf on MFMA results
 # needs no operand quieting: -fno-honor-nans drops one instruction per score.
 EXTRA_FLAGS = {"attn_decode.hip": ["-fno-honor-nans", "-Rpass-analysis=kernel-resource-usage"],
+               "attn_decode_small.hip": ["-fno-honor-nans",
+                                         "-Rpass-analysis=kernel-resource-usage"],
                "attn_prefill.hip": ["-fno-honor-nans", "-Rpass-analysis=kernel-resource-usage"],
                "attn_prefill_f32.hip": ["-fno-honor-nans",
                                         "-Rpass-analysis=kernel-resource-usage"]}
@@ -55,6 +57,7 @@ EXTRA_FLAGS = {"attn_decode.hip": ["-fno-honor-nans", "-Rpass-analysis=kernel-re
 # whose attention kernels use scratch is refused.
 NO_SCRATCH = {"attn_prefill.hip": ("paged_prefill_tiled", "paged_mixed_stream"),
               "attn_decode.hip": ("paged_decode_stream",),
+              "attn_decode_small.hip": ("paged_decode_small",),
               "attn_prefill_f32.hip": ("paged_prefill_f32",)}
 
 

@@ -1,6 +1,7 @@
 // C ABI of paged attention: one varlen call covers decode rows (len_q == 1)
 // and chunked-prefill rows (len_q > 1), dispatched to
-//  * the persistent MFMA decode stream (attn_decode.hip) for decode rows,
+//  * the persistent MFMA decode stream (attn_decode.hip) for decode rows, or
+//    for few short contexts a workgroup per row (attn_decode_small.hip),
 //  * the MFMA prefill kernel (attn_prefill.hip) for prefill rows,
 // when the pool is bf16/f16 with head_dim 64, 128 or 256, a power-of-two
 // block_size >= 16 and at most 16 query heads per kv head (up to 64 when a
@@ -30,25 +31,28 @@ static uint32_t decode_group_parts(uint32_t G) {
 }
 
 // An f32 pool whose calls run on MFMAs: decode rows on the decode stream,
-// prefill rows on the f32 prefill kernels. A small pure-decode call
-// (at most 512 keys per sequence and 8,192 over the batch, config 0's shape)
-// runs the VALU kernel instead, in one launch with no merge. Replayed from
-// a graph, 16 q / 8 kv heads: config 0 (8 x <= 512 keys) 14.1 against
-// 16.4 us; 16 x 128 10.8 against 14.5; 64 x 256 27.3 against 26.3 and
-// 32 x 512 29.2 against 25.8, where the decode stream takes over.
+// prefill rows on the f32 prefill kernels. A small pure-decode call (at most
+// 512 keys per sequence and 8,192 over the batch, config 0's shape) that the
+// short-context decode does not take runs the VALU kernel instead. Replayed
+// from a graph against the stream, 16 q / 8 kv heads: 64 x 256 27.3 against
+// 26.3 us, where the stream takes over; 16 x 128 10.8 against 14.5.
 constexpr uint32_t kSmallKeys = 512;
 constexpr uint64_t kSmallBatchKeys = 8192;
-static bool f32_mfma_ok(const vapi_kv_pool* p, uint32_t num_heads, uint32_t max_q,
-                        uint32_t max_k, uint32_t batch) {
+static bool f32_shape_ok(const vapi_kv_pool* p, uint32_t num_heads) {
   if (p->dtype != VAPI_KV_F32) return false;
-  if (max_q <= 1 && max_k <= kSmallKeys && (uint64_t)batch * max_k <= kSmallBatchKeys)
-    return false;
   // head_dim 64 or 128, or a multiple of 4 below 128 run at the next of
   // them (elements past head_dim read as zeros and never stored).
   if (p->head_dim == 0 || p->head_dim % 4 || p->head_dim > 128) return false;
   if (p->block_size < 16 || (p->block_size & (p->block_size - 1))) return false;
   if (num_heads == 0 || num_heads % p->num_kv_heads) return false;
   return decode_group_parts(num_heads / p->num_kv_heads) > 0;
+}
+
+static bool f32_mfma_ok(const vapi_kv_pool* p, uint32_t num_heads, uint32_t max_q,
+                        uint32_t max_k, uint32_t batch) {
+  if (max_q <= 1 && max_k <= kSmallKeys && (uint64_t)batch * max_k <= kSmallBatchKeys)
+    return false;
+  return f32_shape_ok(p, num_heads);
 }
 
 static bool mfma_ok(const vapi_kv_pool* p, uint32_t num_heads) {
@@ -504,7 +508,14 @@ static int paged_attention_impl(const vapi_kv_pool* pool, uint32_t layer, const 
       a.pf_min_q = 1;
     } else {
       dec.num_waves = a.num_waves;
-      launch_decode(dec, workspace, D, pool->dtype, s);
+      // (The partials lie past the balance block, as the stream's.)
+      const SmallPlan small =
+          decode_small_plan(batch, dec.kvh, dec.group, D, pool->dtype, max_seqlen_k, a.wl,
+                            need - kDecodeBalanceBytes);
+      if (small.ok)
+        launch_decode_small(dec, D, pool->dtype, small, (char*)workspace + kDecodeBalanceBytes, s);
+      else
+        launch_decode(dec, workspace, D, pool->dtype, s);
     }
     if (max_seqlen_q > 1 && pf_n > 0) {
       // The workspace past the decode's part serves the prefill's key split
@@ -518,7 +529,14 @@ static int paged_attention_impl(const vapi_kv_pool* pool, uint32_t layer, const 
       a.pf_min_q = 1;
     } else {
       dec.num_waves = decode_num_waves();
-      launch_decode(dec, workspace, decode_dim(g.d), pool->dtype, s);
+      const SmallPlan small =
+          decode_small_plan(batch, dec.kvh, dec.group, decode_dim(g.d), pool->dtype, max_seqlen_k,
+                            a.wl, need - kDecodeBalanceBytes);
+      if (small.ok)
+        launch_decode_small(dec, decode_dim(g.d), pool->dtype, small,
+                            (char*)workspace + kDecodeBalanceBytes, s);
+      else
+        launch_decode(dec, workspace, decode_dim(g.d), pool->dtype, s);
     }
     if (max_seqlen_q > 1 && pf_n > 0) {
       // The workspace past the decode's part (never its first 256 bytes,
@@ -530,6 +548,18 @@ static int paged_attention_impl(const vapi_kv_pool* pool, uint32_t layer, const 
                          room ? workspace_bytes - off : 0, s);
     }
   } else {
+    // (A small f32 decode: its partials too lie past the balance block.)
+    SmallPlan small{false, 1};
+    if (max_seqlen_q <= 1 && f32_shape_ok(pool, num_heads))
+      small = decode_small_plan(batch, dec.kvh, dec.group, decode_dim(g.d), pool->dtype,
+                                max_seqlen_k, a.wl,
+                                need > kDecodeBalanceBytes ? need - kDecodeBalanceBytes : 0);
+    if (small.ok) {
+      launch_decode_small(dec, decode_dim(g.d), pool->dtype, small,
+                          (char*)workspace + kDecodeBalanceBytes, s);
+      VK_LAUNCHED("paged_attention");
+      return 0;
+    }
     if (g.d > 256)
       VK_FAIL(VAPI_KV_EUNSUP, "vapi_paged_attention: head_dim %u > 256", g.d);
     if (generic_grid(batch, g.kvh, num_heads / g.kvh, max_seqlen_q, max_seqlen_k) > 0xFFFFFFFFull)

@@ -186,6 +186,15 @@ __device__ __forceinline__ bool prefill_item(const AttnArgs& a, const uint32_t* 
   return true;
 }
 
+// This wave's LDS operations are done; then the same for the workgroup (and,
+// unlike __syncthreads(), without waiting for loads in flight into LDS).
+__device__ __forceinline__ void wait_lds() {
+  __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+__device__ __forceinline__ void lds_barrier() {
+  __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 // ---------------------------------------------------------------------------
 // MFMA helpers
 // ---------------------------------------------------------------------------
@@ -705,6 +714,21 @@ size_t decode_workspace_bytes(uint32_t batch, uint32_t kvh, uint32_t group,
                               uint32_t head_dim, uint32_t num_waves);
 void launch_decode(AttnArgs a, void* workspace, uint32_t head_dim, uint32_t dtype,
                    hipStream_t s);
+// The same rows for short contexts (attn_decode_small.hip): workgroups of
+// each (sequence, kv head), n_split of them if its keys are split (then a
+// merge launch follows).
+struct SmallPlan {
+  bool ok;
+  uint32_t n_split;
+};
+// Whether and how a call takes it: kvh and group as the decode counts them,
+// max_k the host's bound on the keys, wl the left window or -1; partials of a
+// split must fit part_bytes.
+SmallPlan decode_small_plan(uint32_t batch, uint32_t kvh, uint32_t group, uint32_t head_dim,
+                            uint32_t dtype, uint32_t max_k, int32_t wl, size_t part_bytes);
+// `part`: the split's partials (16-byte aligned; unused without a split).
+void launch_decode_small(const AttnArgs& a, uint32_t head_dim, uint32_t dtype, SmallPlan plan,
+                         void* part, hipStream_t s);
 // Prefill rows (len_q > 1); bf16/f16, head_dim 64, 128 or 256.
 // Workgroups of the prefill launch (query tiles x kv heads x sequences); a
 // launch needs it below 2^32.

@@ -71,6 +71,21 @@ __device__ __forceinline__ uint32_t decode_steps(const AttnArgs& a,
   return (uint32_t)(len_k - (lo & ~31) + 31) >> 5;
 }
 
+// Fused append: whether decode row s's new key (position len_k - 1) comes
+// from token cu_q[s] of the new rows: if that token's slot is the one the
+// block table gives the position; otherwise the pool is read.
+__device__ __forceinline__ uint32_t fused_row(const AttnArgs& a, const uint32_t* __restrict__ cu_q,
+                                              const uint32_t* __restrict__ cu_k,
+                                              const uint32_t* __restrict__ table, uint32_t s) {
+  const uint32_t q0 = cu_q[s], last = cu_k[s + 1] - cu_k[s] - 1;
+  const uint32_t slot = q0 < a.n_new ? a.slots[q0] : 0xFFFFFFFFu;
+  // Column clamped like every other table read: len_k past the row's
+  // max_blocks * block_size reads the row's last entry.
+  const uint32_t blk =
+      table[(uint64_t)s * a.max_blocks + min(last >> a.bs_shift, a.max_blocks - 1)];
+  return slot < a.num_slots && slot == blk * a.block_size + (last & (a.block_size - 1));
+}
+
 // Waves in group x.
 __device__ __forceinline__ uint32_t group_waves(uint32_t nwg, uint32_t x) {
   return nwg > x ? ((nwg - 1 - x) / kGroups + 1) * kDecodeWavesPerWG : 0u;
@@ -338,22 +353,7 @@ __device__ __forceinline__ void decode_stream_body(const AttnArgs& a,
       P[s] = run;
       const uint32_t ns = decode_steps(a, cu_q, cu_k, s);
       run += ns * kvh_plan;
-      if (kFuse) {
-        // The row's new key (position len_k - 1) comes from token cu_q[s]
-        // of the new rows if that token's slot is the one the block table
-        // gives the position; otherwise the pool is read.
-        uint32_t f = 0;
-        if (ns) {
-          const uint32_t q0 = cu_q[s], last = cu_k[s + 1] - cu_k[s] - 1;
-          const uint32_t slot = q0 < a.n_new ? a.slots[q0] : 0xFFFFFFFFu;
-          // Column clamped like every other table read: len_k past the row's
-          // max_blocks * block_size reads the row's last entry.
-          const uint32_t blk =
-              table[(uint64_t)s * a.max_blocks + min(last >> a.bs_shift, a.max_blocks - 1)];
-          f = slot < a.num_slots && slot == blk * a.block_size + (last & (a.block_size - 1));
-        }
-        FZ[s] = f;
-      }
+      if (kFuse) FZ[s] = ns ? fused_row(a, cu_q, cu_k, table, s) : 0u;
     }
     if (tid == NT - 1) P[B] = run;
     __syncthreads();

@@ -61,13 +61,4 @@ __device__ __forceinline__ uint32_t lds_addr(const uint16_t* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint16_t*)p;
 }
 
-// This wave's LDS operations are done; then the same for the workgroup (and,
-// unlike __syncthreads(), without waiting for loads in flight into LDS).
-__device__ __forceinline__ void wait_lds() {
-  __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-}
-__device__ __forceinline__ void lds_barrier() {
-  __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 }  // namespace vk
