@@ -6,6 +6,8 @@ which they get privately, and which (src, dst) pairs the backend must copy.
 """
 import itertools
 
+import pytest
+
 from vapi_amd.backend import fork_copy_pairs
 
 BS = 4
@@ -63,3 +65,24 @@ def test_pairs_never_overlap_so_one_copy_launch_covers_a_fork():
         dsts = [d for _, d in pairs]
         assert not srcs & set(dsts) and len(dsts) == len(set(dsts))
         assert len(pairs) == (4 if computed % BS else 0)
+
+
+def test_pairs_in_any_form_flatten_to_the_same_ids():
+    """copy_blocks takes what int() takes, from any iterable of pairs."""
+    import numpy as np
+    import torch
+
+    from vapi_amd.backend import _flat_pairs
+    want = [3, 1, 2, 40]
+    pairs = [(3, 1), (2, 40)]
+    for form in (pairs, tuple(pairs), [list(p) for p in pairs], iter(pairs), zip([3, 2], [1, 40]),
+                 np.array(pairs), np.array(pairs, dtype=np.uint32), torch.tensor(pairs),
+                 [(3.0, 1), (2.9, "40")], [(np.uint8(3), True), (np.int64(2), 40)],
+                 {3: 1, 2: 40}.items()):
+        assert list(_flat_pairs(form)) == want
+    assert len(_flat_pairs([])) == 0
+    assert _flat_pairs([(1, 1 << 80)]) == [1, 1 << 80]
+    with pytest.raises(ValueError):
+        _flat_pairs([(1, 2, 3)])
+    with pytest.raises(TypeError):
+        _flat_pairs([(1, None)])

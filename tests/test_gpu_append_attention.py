@@ -153,3 +153,22 @@ def test_fused_step_over_more_rows_than_one_launch_plans_for():
     c, q, batch = random_case(rng, torch.bfloat16, 8, 2, 128, 16, [1] * 5000, lens_k, "HND")
     k_new, v_new = new_rows(5000, 2, 128, torch.bfloat16, 5002)
     check_step(c, q, batch, k_new, v_new, step_slots(batch, 16), same_splits=False)
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.float32, 128)])
+def test_a_decode_grows_a_workspace_that_is_too_small(dtype, d):
+    """The library refuses the small one before it writes anything."""
+    rng = np.random.default_rng(5)
+    lens_k = [900, 40, 3000]
+    c, q, batch = random_case(rng, dtype, 8, 2, d, 16, [1] * 3, lens_k, "HND")
+    k_new, v_new = new_rows(3, 2, d, dtype, 6)
+    s = dev_slots(step_slots(batch, 16))
+    prep = PreparedAttention.from_batch(batch, DEV)
+    want = paged_attention_append_prepared(q, k_new, v_new, s, c, 0, prep, d ** -0.5)
+    size = prep.workspace.numel()
+    for fn in (lambda p: paged_attention_append_prepared(q, k_new, v_new, s, c, 0, p, d ** -0.5),
+               lambda p: paged_attention_prepared(q, c, 0, p, d ** -0.5)):
+        small = PreparedAttention.from_batch(batch, DEV)
+        small.workspace = torch.zeros(256, dtype=torch.uint8, device=DEV)
+        assert torch.equal(fn(small), want)
+        assert small.workspace.numel() == size

@@ -233,6 +233,28 @@ def test_copy_blocks_rejects_overlapping_pairs():
         KvBlockBackend(c).copy_blocks([(1, 2), (2, 3)])
     with pytest.raises(ValueError):
         KvBlockBackend(c).copy_blocks([(1, 8)])
+    with pytest.raises(ValueError, match="block -1 of 8"):
+        KvBlockBackend(c).copy_blocks([(1, -1), (9, 2)])
+    with pytest.raises(ValueError, match="block 1208925819614629174706176 of 8"):
+        KvBlockBackend(c).copy_blocks([(1, 1 << 80)])
+
+
+def test_back_to_back_copies_on_two_streams_see_their_streams_earlier_work():
+    """copy_blocks does not wait for the GPU: each call's pairs still reach
+    the launch they belong to, on the current stream and on a given one."""
+    side = torch.cuda.Stream()
+    for stream in (None, side):
+        c = PagedKvCache(2, 400, 16, 4, 128, torch.bfloat16)
+        for l in range(2):
+            c.k[l][0] = l + 1.0
+            c.v[l][0] = l + 5.0
+        torch.cuda.synchronize()
+        b = KvBlockBackend(c)
+        for i in range(1, 400):  # a chain: call i reads what call i - 1 wrote
+            b.copy_blocks([(i - 1, i)], stream=stream)
+        torch.cuda.synchronize()
+        for l in range(2):
+            assert bool((c.k[l] == l + 1.0).all()) and bool((c.v[l] == l + 5.0).all())
 
 
 @pytest.mark.parametrize("layout", LAYOUTS)

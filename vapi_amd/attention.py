@@ -14,7 +14,7 @@ from dataclasses import dataclass, field
 import numpy as np
 import torch
 
-from ._lib import check, lib
+from ._lib import ESPACE, check, lib
 from .cache import PagedKvCache, _per_layer, stream_handle
 
 _u32p = ctypes.POINTER(ctypes.c_uint32)
@@ -181,6 +181,22 @@ def _workspace(cache, prepared: PreparedAttention, b: int, num_heads: int, max_q
     return need, ws
 
 
+def _run(call, cache, prepared: PreparedAttention, b: int, num_heads: int, max_q: int,
+         max_k: int, device) -> None:
+    """call(workspace pointer, bytes) with the step's workspace, grown first
+    if it is too small. A decode's workspace has no optional part, so the
+    library, which refuses a small one before it launches anything, is asked
+    first (the size query is ~1 us of a call's ~8)."""
+    ws = prepared.workspace
+    if max_q == 1 and ws is not None:
+        rc = call(ws.data_ptr(), ws.numel())
+        if rc != ESPACE:
+            check(rc)
+            return
+    need, ws = _workspace(cache, prepared, b, num_heads, max_q, max_k, device)
+    check(call(ws.data_ptr() if need else None, need))
+
+
 def paged_attention_prepared(q: torch.Tensor, cache: PagedKvCache, layer: int,
                              prepared: PreparedAttention, softmax_scale: float,
                              window_size_left: int | None = None,
@@ -202,18 +218,19 @@ def paged_attention_prepared(q: torch.Tensor, cache: PagedKvCache, layer: int,
     num_heads = q.shape[1]
     max_q = max(int(prepared.max_seqlen_q), 1)
     max_k = max(int(prepared.max_seqlen_k), 1)
-    need, ws = _workspace(cache, prepared, b, num_heads, max_q, max_k, q.device)
     args = (cache.pool, layer, q.data_ptr(), out.data_ptr(), prepared.seqlens_q.data_ptr(),
             prepared.seqlens_k.data_ptr(), prepared.block_table.data_ptr(), b,
             prepared.block_table.shape[1], max_q, max_k, num_heads, float(softmax_scale),
             -1 if window_size_left is None else int(window_size_left),
             -1 if window_size_right is None else int(window_size_right), prepared.flags)
-    tail = (ws.data_ptr() if need else None, need, stream_handle(stream))
+    handle = stream_handle(stream)
     if prepared.prefill_seqs is None:
-        check(lib().vapi_paged_attention_ex(*args, *tail))
+        fn = lib().vapi_paged_attention_ex
     else:
-        check(lib().vapi_paged_attention_prepared(
-            *args, prepared.prefill_seqs.data_ptr(), prepared.n_prefill, *tail))
+        fn = lib().vapi_paged_attention_prepared
+        args += (prepared.prefill_seqs.data_ptr(), prepared.n_prefill)
+    _run(lambda ptr, size: fn(*args, ptr, size, handle), cache, prepared, b, num_heads, max_q,
+         max_k, q.device)
     return out
 
 
@@ -255,8 +272,8 @@ def paged_attention_append_prepared(q: torch.Tensor, k: torch.Tensor, v: torch.T
         raise ValueError(f"q must be (tokens, heads, {cache.head_dim}), got {tuple(q.shape)}")
     if q.dtype != cache.dtype or k.dtype != cache.dtype or v.dtype != cache.dtype:
         raise ValueError(f"q/k/v must be {cache.dtype}")
-    if tuple(k.shape) != tuple(v.shape) or k.dim() != 3 or \
-            tuple(k.shape[1:]) != (cache.num_kv_heads, cache.head_dim):
+    if k.shape != v.shape or k.dim() != 3 or \
+            k.shape[1:] != (cache.num_kv_heads, cache.head_dim):
         raise ValueError(f"k/v must be (n, {cache.num_kv_heads}, {cache.head_dim}), "
                          f"got {tuple(k.shape)} and {tuple(v.shape)}")
     if slot_mapping.numel() != k.shape[0] or slot_mapping.element_size() != 4:
@@ -279,13 +296,13 @@ def paged_attention_append_prepared(q: torch.Tensor, k: torch.Tensor, v: torch.T
         return paged_attention_prepared(q, cache, layer, prepared, softmax_scale,
                                         window_size_left, window_size_right, out=out,
                                         stream=stream)
-    need, ws = _workspace(cache, prepared, b, num_heads, max_q, max_k, q.device)
-    check(lib().vapi_paged_attention_append_ex(
-        cache.pool, layer, k.data_ptr(), v.data_ptr(), slot_mapping.data_ptr(), k.shape[0],
-        q.data_ptr(), out.data_ptr(), prepared.seqlens_q.data_ptr(),
-        prepared.seqlens_k.data_ptr(), prepared.block_table.data_ptr(), b,
-        prepared.block_table.shape[1], max_q, max_k, num_heads, float(softmax_scale),
-        -1 if window_size_left is None else int(window_size_left),
-        -1 if window_size_right is None else int(window_size_right), prepared.flags,
-        ws.data_ptr() if need else None, need, stream_handle(stream)))
+    args = (cache.pool, layer, k.data_ptr(), v.data_ptr(), slot_mapping.data_ptr(), k.shape[0],
+            q.data_ptr(), out.data_ptr(), prepared.seqlens_q.data_ptr(),
+            prepared.seqlens_k.data_ptr(), prepared.block_table.data_ptr(), b,
+            prepared.block_table.shape[1], max_q, max_k, num_heads, float(softmax_scale),
+            -1 if window_size_left is None else int(window_size_left),
+            -1 if window_size_right is None else int(window_size_right), prepared.flags)
+    handle, fn = stream_handle(stream), lib().vapi_paged_attention_append_ex
+    _run(lambda ptr, size: fn(*args, ptr, size, handle), cache, prepared, b, num_heads, max_q,
+         max_k, q.device)
     return out

@@ -20,6 +20,40 @@ def _dev_u32(values, device) -> torch.Tensor:
     return torch.from_numpy(a.view(np.int32)).to(device)
 
 
+def _dev_u32_async(values: np.ndarray, device) -> torch.Tensor:
+    """_dev_u32 on the current stream without waiting for it: through pinned
+    memory from torch's caching allocator, which reuses it only once the copy
+    has run. (A copy from pageable memory waits for the stream's earlier work,
+    so a burst of calls leaves the GPU idle in between.) Where the copy would
+    not be on the current stream, or that stream is being captured, _dev_u32:
+    the capture refuses its copy, where a recorded one would read the buffer
+    again on every replay."""
+    device = torch.device(device)
+    if (device.type != "cuda" or torch.cuda.is_current_stream_capturing() or
+            device.index not in (None, torch.cuda.current_device())):
+        return _dev_u32(values, device)
+    host = torch.empty(len(values), dtype=torch.int32, pin_memory=True)
+    host.numpy()[:] = values.astype(np.uint32).view(np.int32)
+    return host.to(device, non_blocking=True)
+
+
+def _flat_pairs(pairs) -> list | np.ndarray:
+    """(source, destination) pairs one after the other, as int64; as a list
+    of ints if one of them does not fit."""
+    flat = [x for s, d in pairs for x in (s, d)]
+    try:
+        a = np.array(flat)
+        if a.ndim == 1 and a.dtype.kind == "i":
+            return a.astype(np.int64, copy=False)
+    except (TypeError, ValueError, RuntimeError):  # not plain numbers
+        pass
+    flat = [int(x) for x in flat]
+    try:
+        return np.array(flat, dtype=np.int64)
+    except OverflowError:
+        return flat
+
+
 class KvBlockBackend:
     """The block-moving half of a backend over one PagedKvCache."""
 
@@ -82,16 +116,18 @@ class KvBlockBackend:
     def copy_blocks(self, pairs, stream=None) -> None:
         """Copy-on-write (backend.rs:781-797): every pair, every layer, K and V,
         in one launch. A destination must not be another pair's source."""
-        pairs = [(int(s), int(d)) for s, d in pairs]
-        if not pairs:
+        flat = _flat_pairs(pairs)
+        n = len(flat) // 2
+        if n == 0:
             return
-        self._check_ids([x for p in pairs for x in p])
-        srcs = {s for s, _ in pairs}
-        dsts = [d for _, d in pairs]
-        if len(set(dsts)) != len(dsts) or srcs.intersection(dsts):
+        if isinstance(flat, list) or flat.min() < 0 or flat.max() >= self.cache.num_blocks:
+            self._check_ids(flat)  # names the first one out of range
+        dsts = flat[1::2].tolist()
+        if len(set(dsts)) != n or not set(flat[::2].tolist()).isdisjoint(dsts):
             raise ValueError("copy_blocks: destinations must be distinct and not sources")
-        d_pairs = _dev_u32([x for p in pairs for x in p], self.cache.device)
-        check(lib().vapi_kv_copy_blocks(self.cache.pool, d_pairs.data_ptr(), len(pairs),
+        with torch.cuda.stream(stream):  # (None: the current stream)
+            d_pairs = _dev_u32_async(flat, self.cache.device)
+        check(lib().vapi_kv_copy_blocks(self.cache.pool, d_pairs.data_ptr(), n,
                                         stream_handle(stream)))
 
     def swap_out(self, ids_dev: torch.Tensor, host: torch.Tensor, staging: torch.Tensor,

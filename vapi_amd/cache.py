@@ -30,9 +30,18 @@ def dtype_code(dt: torch.dtype) -> int:
         raise TypeError(f"unsupported KV dtype {dt}") from None
 
 
+# The current stream's handle without building a torch.cuda.Stream for it
+# (~0.2 against ~2.5 us, in calls of 5-12 us). Absent in builds without GPU
+# support, where torch.cuda.current_stream() raises its own error.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(stream=None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch._C._cuda_getDevice())
 
 
 class PagedKvCache:
