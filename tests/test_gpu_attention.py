@@ -865,3 +865,40 @@ def test_keys_outside_a_short_decodes_range_do_not_reach_its_output(dtype):
             c.k[0][t[pos // 16], :, pos % 16] = float("inf")
             c.v[0][t[pos // 16], :, pos % 16] = -float("inf")
     assert torch.equal(paged_attention_prepared(q, c, 0, prep, 128 ** -0.5, 20), want)
+
+
+# ---- prefill launches cut into ranges of equal work -----------------------------
+
+RANGE_CASES = [
+    # dtype, heads, kvh, d, bs, lens_q, lens_k, window, layout
+    (torch.bfloat16, 8, 2, 128, 16, [700, 40, 300], [9000, 4000, 2500], None, "HND"),
+    (torch.float16, 7, 1, 128, 32, [300, 301], [8000, 301], None, "NHD"),
+    (torch.bfloat16, 8, 8, 64, 16, [520, 3, 256], [9100, 9100, 256], None, "HND"),
+    (torch.bfloat16, 8, 4, 96, 16, [600, 90, 700], [7000, 6100, 6000], 4000, "HND"),
+    (torch.bfloat16, 4, 1, 128, 16, [33] * 64, [6000] + [400] * 63, None, "HND"),
+    (torch.float32, 8, 4, 128, 16, [130, 70, 200], [4000, 900, 3100], None, "HND"),
+    (torch.float32, 8, 2, 80, 16, [100, 150, 17], [3000, 3000, 2500], 1500, "NHD"),
+    (torch.float32, 4, 2, 64, 32, [17] * 40, [2000] * 5 + [100] * 35, None, "HND"),
+]
+
+
+@pytest.mark.parametrize("case", RANGE_CASES,
+                         ids=lambda c: f"{str(c[0])[6:]}-g{c[1] // c[2]}-d{c[3]}-n{len(c[5])}-w{c[7]}")
+def test_prefill_in_ranges_of_equal_work_matches_the_oracle(case):
+    """Lengths whose tiles leave the GPU idle: ranges that end inside tiles,
+    cover several and span kv heads; with decode rows beside them too, and
+    against the same call unsplit (deterministic)."""
+    dtype, heads, kvh, d, bs, lens_q, lens_k, window, layout = case
+    rng = np.random.default_rng(zlib.crc32(str(case).encode()))
+    left = None if window is None else window - 1
+    for rows in (lens_q, [1] + lens_q[1:]):
+        c, q, batch = random_case(rng, dtype, heads, kvh, d, bs, rows, lens_k, layout)
+        want = oracle_out(q, c, 0, batch, d ** -0.5, window)
+        tol = (1e-5 if dtype == torch.float32 else
+               (2e-2 if dtype == torch.bfloat16 else 1e-2) * float(want.abs().max()))
+        for det in (False, True):
+            prep = PreparedAttention.from_batch(batch, DEV, cache=c, num_heads=heads,
+                                                deterministic=det)
+            got = torch.full_like(q, float("nan"))
+            paged_attention_prepared(q, c, 0, prep, d ** -0.5, left, out=got)
+            assert max_abs(got, want) <= tol

@@ -111,21 +111,17 @@ __device__ __forceinline__ void lgkm_wait(uint2 (&r)[4]) {
 }
 
 
-// With n_split > 1 the keys a workgroup would walk are cut into n_split
-// contiguous runs of steps, one workgroup each (a batch too small to fill
-// the GPU with query tiles alone); each writes its rows' (m, l, o) to
-// `part` and paged_prefill_merge combines them.
-// Workgroup `bid` (W waves) of a prefill launch.
+// One item (W waves): query tile it.qt of a sequence and kv head. kSplit 0:
+// all of it, to the output (compiled without the shares' arithmetic); 1: its
+// steps [u0, u1) of c shares, the rows' (m, l, o) to the partial `pb`; 2: the
+// same, or to the output if pb is null (all of the item: u0 = 0, u1 = c).
 // DL: the 16-column d tiles that hold head_dim (kPad; D / 16 otherwise):
 // the score MFMAs, V^T reads, PV MFMAs and stores of the tiles past them
 // are left out.
-template <typename T, int D, int RT, int W, bool kSplit, bool kPad = false, int DL = D / 16>
-__device__ __forceinline__ void prefill_body(
-    const AttnArgs& a, const uint32_t* __restrict__ cu_q, const uint32_t* __restrict__ cu_k,
-    const uint32_t* __restrict__ table, uint32_t qtiles, uint32_t n_split_arg,
-    float* __restrict__ part, uint32_t bid) {
-  // The unsplit launch compiles without the split's arithmetic.
-  const uint32_t n_split = kSplit ? n_split_arg : 1u;
+template <typename T, int D, int RT, int W, int kSplit, bool kPad = false, int DL = D / 16>
+__device__ __forceinline__ void prefill_piece(const AttnArgs& a, const uint32_t* __restrict__ table,
+                                              const PfItem& it, uint32_t u0, uint32_t u1,
+                                              uint32_t c, char* pb) {
   static_assert(W == 8 || W == 4, "a step's K and V are loaded by 8 or 4 waves");
   constexpr int KC = D / 32;
   constexpr int DT = D / 16;  // 16-column d tiles
@@ -142,15 +138,7 @@ __device__ __forceinline__ void prefill_body(
   // every LDS read.
   __shared__ __attribute__((aligned(16))) uint16_t k0[32 * D], k1[32 * D], k2[32 * D];
   __shared__ __attribute__((aligned(16))) uint16_t v0[32 * D], v1[32 * D], v2[32 * D];
-  // Item order: kv head fastest, then key split, then query tile (the split
-  // index counts per tile, so the items of one tile stay together).
-  __shared__ uint32_t order[64 * W];
-  const uint32_t hr = bid / a.kvh, split = hr % n_split;
-  PfItem it;
-  if (!prefill_item<W>(a, cu_q, cu_k, (hr / n_split) * a.kvh + bid % a.kvh, qtiles, kPfRows,
-                       order, it))
-    return;
-  const uint32_t qt = it.qt, kh = it.kh, seq = it.seq, rest = it.li * a.kvh + kh;
+  const uint32_t qt = it.qt, kh = it.kh, seq = it.seq;
   const uint32_t q0 = it.q0, len_q = it.len_q;
   const uint32_t G = a.group;
   const uint32_t nrows = len_q * G;
@@ -168,12 +156,12 @@ __device__ __forceinline__ void prefill_body(
   const int32_t wg_pmax = offset + (int32_t)(wg_last / G);
   const int32_t klo_wg = a.wl >= 0 ? max(0, wg_pmin - a.wl) : 0;
   const int32_t khi_wg = a.wr >= 0 ? min(last, wg_pmax + a.wr) : last;
-  // This workgroup's run of 32-key steps: all of them, or split's share.
+  // This workgroup's run of 32-key steps: all of them, or its share.
   int32_t klo = klo_wg, khi = khi_wg;
   if (kSplit) {
     const int32_t first = klo_wg & ~31;
     const uint32_t steps = khi_wg >= klo_wg ? (uint32_t)(((khi_wg & ~31) - first) / 32 + 1) : 0u;
-    const uint32_t a0 = split * steps / n_split, a1 = (split + 1) * steps / n_split;
+    const uint32_t a0 = pf_step_at(u0, c, steps), a1 = pf_step_at(u1, c, steps);
     klo = max(klo_wg, first + 32 * (int32_t)a0);
     khi = min(khi_wg, first + 32 * (int32_t)a1 - 1);  // < klo when the share is empty
   }
@@ -353,13 +341,10 @@ __device__ __forceinline__ void prefill_body(
   }
   wait_vmcnt<0>();  // no load may land in LDS after the workgroup ends
 
-  if constexpr (kSplit) {
-    // Partials of this split (pf_part_bytes per item and split): per row
-    // (m in scaled log2 units, l) as f32, then per row o / l as f32 (the
-    // merge weighs it by l). An empty share leaves l = 0 and its o
-    // unwritten.
-    char* pb = (char*)part + ((uint64_t)(rest * qtiles + qt) * n_split + split) *
-                                 pf_part_bytes(kPfRows, D);
+  if (kSplit == 1 || (kSplit == 2 && pb)) {
+    // The partial (pf_part_bytes): per row (m in scaled log2 units, l) as
+    // f32, then per row o / l as f32 (the merge weighs it by l). An empty
+    // share leaves l = 0 and its o unwritten.
 #pragma unroll
     for (int t = 0; t < kPfRT; ++t) {
       const float lt = wave_sum_g(l_run[t]);
@@ -391,6 +376,30 @@ __device__ __forceinline__ void prefill_body(
   }
 }
 
+// Workgroup `bid` of a prefill launch. With n_split > 1 the steps of each
+// item are cut into n_split equal runs, one workgroup each, and
+// paged_prefill_merge combines their partials. Item order: kv head fastest,
+// then key split, then query tile (the items of one tile stay together).
+template <typename T, int D, int RT, int W, bool kSplit, bool kPad = false, int DL = D / 16>
+__device__ __forceinline__ void prefill_body(
+    const AttnArgs& a, const uint32_t* __restrict__ cu_q, const uint32_t* __restrict__ cu_k,
+    const uint32_t* __restrict__ table, uint32_t qtiles, uint32_t n_split_arg,
+    float* __restrict__ part, uint32_t bid) {
+  constexpr uint32_t kRows = 16 * RT * W;
+  const uint32_t n_split = kSplit ? n_split_arg : 1u;
+  __shared__ uint32_t order[64 * W];
+  const uint32_t hr = bid / a.kvh, split = hr % n_split;
+  PfItem it;
+  if (!prefill_item<W>(a, cu_q, cu_k, (hr / n_split) * a.kvh + bid % a.kvh, qtiles, kRows, order,
+                       it))
+    return;
+  char* pb = nullptr;
+  if (kSplit)
+    pb = (char*)part + ((uint64_t)((it.li * a.kvh + it.kh) * qtiles + it.qt) * n_split + split) *
+                           pf_part_bytes(kRows, D);
+  prefill_piece<T, D, RT, W, kSplit ? 1 : 0, kPad, DL>(a, table, it, split, split + 1, n_split, pb);
+}
+
 template <typename T, int D, int RT, int OCC, bool kSplit, bool kPad, int DL = D / 16>
 __global__ __launch_bounds__(kPfThreads, OCC) void paged_prefill_tiled(
     AttnArgs a, const uint32_t* __restrict__ cu_q, const uint32_t* __restrict__ cu_k,
@@ -400,32 +409,43 @@ __global__ __launch_bounds__(kPfThreads, OCC) void paged_prefill_tiled(
                                            blockIdx.x);
 }
 
-// Combines the key splits' partials of a prefill launch: thread (row, four
-// consecutive d) over the splits, in split order. Output rows are a.hd
-// elements apart; with a head_dim below D the columns past it are not
-// stored.
-template <typename T, int D>
-__device__ __forceinline__ void prefill_merge_body(const AttnArgs& a, uint32_t qtiles,
-                                                   uint32_t rows_per_item, uint32_t n_split,
-                                                   const float* __restrict__ part,
-                                                   uint32_t bid) {
+// The same over ranges of equal work (see attn_prefill.hpp).
+// (One workgroup per CU at every head_dim: at 64 the walk takes the kernel past
+// the 128 registers of two, which are worth 1%.)
+template <typename T, int D, int RT, bool kPad, int DL = D / 16>
+__global__ __launch_bounds__(kPfThreads, 1) void paged_prefill_tiled_ranges(
+    AttnArgs a, const uint32_t* __restrict__ cu_q, const uint32_t* __restrict__ cu_k,
+    const uint32_t* __restrict__ table, uint32_t qtiles, uint32_t ranges,
+    PfSplitTile* __restrict__ tiles, char* __restrict__ part) {
+  constexpr uint32_t kRows = 16 * RT * kPfWaves;
+  pf_walk_range<kPfWaves>(a, cu_q, cu_k, qtiles, kRows, ranges, tiles, blockIdx.x,
+                [&](const PfItem& it, uint32_t u0, uint32_t u1, uint32_t c, uint32_t slot)
+                    __attribute__((always_inline)) {
+                  prefill_piece<T, D, RT, kPfWaves, 2, kPad, DL>(
+                      a, table, it, u0, u1, c,
+                      slot == ~0u ? nullptr : part + (uint64_t)slot * pf_part_bytes(kRows, D));
+                });
+}
+
+// Combines the n partials of one item: this thread (a row of the item, four
+// consecutive d) over the partials partial(0) .. partial(n - 1), in order.
+// Output rows are a.hd elements apart; with a head_dim below D the columns
+// past it are not stored.
+template <typename T, int D, typename Partial>
+__device__ __forceinline__ void prefill_merge_rows(const AttnArgs& a, uint32_t seq, uint32_t qt,
+                                                   uint32_t kh, uint32_t rows_per_item,
+                                                   uint32_t row_block, uint32_t n_split,
+                                                   Partial partial) {
   constexpr uint32_t kTpr = D / 4;           // threads per row
   constexpr uint32_t kRpw = 256 / kTpr;      // rows per workgroup
-  const uint32_t blocks_per_item = rows_per_item / kRpw;
-  const uint32_t base = bid / blocks_per_item;
-  const uint32_t row_in = (bid % blocks_per_item) * kRpw + threadIdx.x / kTpr;
+  const uint32_t row_in = row_block * kRpw + threadIdx.x / kTpr;
   const uint32_t dq = (threadIdx.x % kTpr) * 4;
-  const uint32_t qt = base % qtiles, rest = base / qtiles;
-  const uint32_t kh = rest % a.kvh;
-  const uint32_t seq = a.pf_seqs ? a.pf_seqs[rest / a.kvh] : rest / a.kvh;
   if (seq >= a.batch) return;
   const uint32_t q0 = a.cu_q[seq], len_q = a.cu_q[seq + 1] - q0;
   if (len_q < a.pf_min_q || len_q == 0) return;
   const uint32_t G = a.group;
   const uint32_t row = qt * rows_per_item + row_in;
   if (row >= len_q * G || dq >= a.hd) return;
-  const uint64_t stride = pf_part_bytes(rows_per_item, D);  // per split
-  const char* p0 = (const char*)part + (uint64_t)base * n_split * stride;
   const uint64_t ml_off = (uint64_t)row_in * 8;
   const uint64_t o_off = (uint64_t)rows_per_item * 8 + ((uint64_t)row_in * D + dq) * sizeof(float);
   // Eight splits per memory round trip: every (m, l) and o load of a batch
@@ -439,7 +459,7 @@ __device__ __forceinline__ void prefill_merge_body(const AttnArgs& a, uint32_t q
 #pragma unroll
     for (uint32_t u = 0; u < kB; ++u) {
       const bool in = s0 + u < n_split;
-      const char* pr = p0 + (uint64_t)(in ? s0 + u : s0) * stride;
+      const char* pr = partial(in ? s0 + u : s0);
       ml[u] = *(const float2*)(pr + ml_off);
       xb[u] = *(const float4*)(pr + o_off);
       if (!in) ml[u].y = 0.f;
@@ -470,6 +490,40 @@ __device__ __forceinline__ void prefill_merge_body(const AttnArgs& a, uint32_t q
     *(float4*)orow = make_float4(o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv);
   else
     *(uint2*)orow = make_uint2(pack2<T>(o[0] * inv, o[1] * inv), pack2<T>(o[2] * inv, o[3] * inv));
+}
+
+// The partials of a launch whose items are all split n_split ways.
+template <typename T, int D>
+__device__ __forceinline__ void prefill_merge_body(const AttnArgs& a, uint32_t qtiles,
+                                                   uint32_t rows_per_item, uint32_t n_split,
+                                                   const float* __restrict__ part,
+                                                   uint32_t bid) {
+  const uint32_t blocks_per_item = rows_per_item / (256 / (D / 4));
+  const uint32_t base = bid / blocks_per_item;
+  const uint32_t rest = base / qtiles, li = rest / a.kvh;
+  const uint64_t stride = pf_part_bytes(rows_per_item, D);
+  const char* p0 = (const char*)part + (uint64_t)base * n_split * stride;
+  prefill_merge_rows<T, D>(a, a.pf_seqs ? a.pf_seqs[li] : li, base % qtiles, rest % a.kvh,
+                           rows_per_item, bid % blocks_per_item, n_split,
+                           [&](uint32_t s) { return p0 + s * stride; });
+}
+
+// Those of a launch of ranges: range r's split tile. (A resident grid that
+// counts the split tiles and loops over them was slower: 3 chunks of 512 over
+// 4,096 keys 134 against 124 us.)
+template <typename T, int D>
+__global__ __launch_bounds__(256) void paged_prefill_range_merge(
+    AttnArgs a, uint32_t rows_per_item, const PfSplitTile* __restrict__ tiles,
+    const char* __restrict__ part) {
+  const uint32_t blocks_per_item = rows_per_item / (256 / (D / 4));
+  const uint32_t r = blockIdx.x / blocks_per_item;
+  const PfSplitTile t = tiles[r];
+  if (!t.valid) return;
+  const uint64_t stride = pf_part_bytes(rows_per_item, D);
+  prefill_merge_rows<T, D>(a, t.seq, t.qt, t.kh, rows_per_item, blockIdx.x % blocks_per_item,
+                           t.last - r + 1, [&](uint32_t s) {
+                             return part + (uint64_t)(s ? 2 * (r + s) : t.first_slot) * stride;
+                           });
 }
 
 template <typename T, int D>
@@ -531,6 +585,80 @@ static uint32_t pf_splits_within(uint64_t base, uint32_t max_k, uint32_t head_di
   while (n > 1 && pf_split_bytes(base, n, head_dim, rows) > std::min(bytes, kPfSplitMaxBytes))
     --n;
   return n;
+}
+
+// Ranges of equal work instead of tiles or their n_split equal shares, where
+// what those leave idle is more than the ranges' plan, partials and merge
+// cost (a partial is written and read once; ~ranges + tiles of them against
+// n_split per tile). The host knows the longest sequence only: idle is what
+// the rounds of workgroups leave if all are as long (5% at least). Measured
+// (us, tiles or shares / ranges; bf16, 32 q / 8 kv heads): 3 x 512 queries
+// over 4,096 keys (192 tiles in 384 shares) 150 / 126, 5 x 512 (320 tiles)
+// 242 / 197, 10 chunks of 20-100 over ~1,000 keys 79 / 53; f32, 40 chunks of
+// 16 over ~1,000 keys 378 / 168; and where it says no: 4 x 512 (256 tiles) 135
+// / 154, 1 x 512 (256 shares) 57 / 63, 1 x 1,500 fresh 53 / 73.
+PfRangePlan pf_range_plan(uint64_t items, uint32_t max_q, uint32_t max_k, uint32_t slots,
+                          uint32_t n_split, float step_us, uint64_t part_bytes,
+                          size_t ws_bytes) {
+  constexpr float kMergeUs = 4.f, kPlanUs = 5.f, kMarginUs = 3.f, kBytesPerUs = 5e6f;
+  PfRangePlan p{0, 0};
+  if (items == 0 || items >= 4 * slots) return p;
+  const uint64_t wgs = items * n_split, rounds = (wgs + slots - 1) / slots;
+  const float idle = std::max(1.f - (float)wgs / (float)(rounds * slots), 0.05f);
+  const float steps_now = (float)(max_k - std::min(max_q / 2, max_k)) / 32.f / (float)n_split;
+  const float part_us = 2.f * (float)part_bytes / kBytesPerUs;
+  const float cost = kPlanUs + kMergeUs + part_us * (float)(kPfMaxRanges + items) -
+                     (n_split > 1 ? kMergeUs + part_us * (float)wgs : 0.f);
+  if ((float)rounds * steps_now * step_us * idle < cost + kMarginUs) return p;
+  // The steps there can be, kPfMinSteps to a range; two partials each.
+  const uint64_t steps = items * (max_k / 32 + 2);
+  if (16 * steps > kPfMaxCount) return p;
+  uint64_t n = std::min<uint64_t>(kPfMaxRanges, (steps + kPfMinSteps - 1) / kPfMinSteps);
+  const uint64_t bytes = std::min<uint64_t>(ws_bytes, kPfSplitMaxBytes);
+  if (bytes <= kPfRangeHead) return p;
+  n = std::min<uint64_t>(n, (bytes - kPfRangeHead) / (2 * part_bytes));
+  if (n < 2) return p;
+  p.ranges = (uint32_t)n;
+  p.bytes = kPfRangeHead + n * 2 * part_bytes;
+  return p;
+}
+
+// Launches that may run as ranges: at head_dim 256 the walk over a range's
+// pieces does not fit beside the kernel's registers, and longer lists do not
+// fit the plan; those split every item equally where they split.
+static bool pf_ranges_ok(uint32_t n_seqs, uint32_t head_dim) {
+  return n_seqs <= kPfSortSeqs && head_dim <= 128;
+}
+
+// A full workgroup's 32-key step (head_dim 128; less below).
+constexpr float kPfStepUs = 1.15f;
+// Workgroups of the tiled prefill that the GPU runs at once.
+static uint32_t pf_slots(uint32_t head_dim) { return 256u * (head_dim == 64 ? kPfOcc64 : kPfOcc); }
+
+void launch_prefill_range_merge(const AttnArgs& a, uint32_t ranges, uint32_t rows, uint32_t dtype,
+                                uint32_t head_dim, const void* ws, hipStream_t s) {
+  const PfSplitTile* tiles = (const PfSplitTile*)ws;
+  const char* part = (const char*)ws + kPfRangeHead;
+#define VK_RM(T, DD)                                                                     \
+  hipLaunchKernelGGL((paged_prefill_range_merge<T, DD>),                                 \
+                     dim3(ranges * (rows / (256 / (DD / 4)))), dim3(256), 0, s, a, rows, \
+                     tiles, part)
+#define VK_RM_D(T)                     \
+  do {                                 \
+    if (head_dim == 256) VK_RM(T, 256); \
+    else if (head_dim == 128) VK_RM(T, 128); \
+    else VK_RM(T, 64);                 \
+  } while (0)
+  if (dtype == VAPI_KV_F32) {
+    if (head_dim == 128) VK_RM(float, 128);
+    else VK_RM(float, 64);
+  } else if (dtype == VAPI_KV_BF16) {
+    VK_RM_D(bf16_t);
+  } else {
+    VK_RM_D(f16_t);
+  }
+#undef VK_RM_D
+#undef VK_RM
 }
 
 // ---- a mixed step in one launch ---------------------------------------------
@@ -662,8 +790,12 @@ size_t prefill_split_bytes(uint32_t batch, uint32_t kvh, uint32_t group, uint32_
   if (max_q <= 1) return 0;
   const uint32_t rows = pf_rows(head_dim);
   const uint64_t base = prefill_grid(batch, kvh, group, max_q, head_dim);
-  return (size_t)pf_split_bytes(base, pf_splits_within(base, max_k, head_dim, ~0ull, rows),
-                                head_dim, rows);
+  const uint32_t n = pf_splits_within(base, max_k, head_dim, ~0ull, rows);
+  const size_t split = (size_t)pf_split_bytes(base, n, head_dim, rows);
+  if (!pf_ranges_ok(batch, head_dim)) return split;
+  return std::max(split, pf_range_plan(base, max_q, max_k, pf_slots(head_dim), n, kPfStepUs,
+                                       pf_part_bytes(rows, head_dim), ~0ull)
+                             .bytes);
 }
 
 void launch_prefill(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, uint32_t head_dim,
@@ -676,16 +808,29 @@ void launch_prefill(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, uint32
   // As many splits as the workspace given holds (none without one); a
   // deterministic call does not split, so its output does not depend on
   // the workspace it is given.
-  const uint32_t n_split = split_ws && !a.deterministic
-                               ? pf_splits_within(base, max_k, head_dim, split_ws_bytes, rows)
-                               : 1;
+  const bool split_ok = split_ws && !a.deterministic;
+  const uint32_t n_split =
+      split_ok ? pf_splits_within(base, max_k, head_dim, split_ws_bytes, rows) : 1;
+  const PfRangePlan rp =
+      split_ok && pf_ranges_ok(a.pf_seqs_n, head_dim)
+          ? pf_range_plan(base, max_q, max_k, pf_slots(head_dim), n_split, kPfStepUs,
+                          pf_part_bytes(rows, head_dim), split_ws_bytes)
+          : PfRangePlan{0, 0};
   float* part = n_split > 1 ? (float*)split_ws : nullptr;
   const dim3 grid((uint32_t)(base * n_split)), block(kPfThreads);
 #define VK_PF(T, DD, PAD, DL)                                                                    \
   do {                                                                                           \
     constexpr int occ = DD == 64 ? kPfOcc64 : kPfOcc;                                            \
     constexpr int rt = DD == 256 ? kPfRowTiles256 : kPfRowTiles;                                 \
-    if (n_split > 1) {                                                                           \
+    if (rp.ranges) {                                                                             \
+      if constexpr (DD <= 128)                                                                   \
+        hipLaunchKernelGGL((paged_prefill_tiled_ranges<T, DD, rt, PAD, DL>),                \
+                           dim3(rp.ranges), block, 0, s, a, a.cu_q, a.cu_k, a.table, qtiles,     \
+                           rp.ranges, (PfSplitTile*)split_ws,                                    \
+                           (char*)split_ws + kPfRangeHead);                                      \
+      launch_prefill_range_merge(a, rp.ranges, rows, bf16 ? VAPI_KV_BF16 : VAPI_KV_F16, DD,      \
+                                 split_ws, s);                                                   \
+    } else if (n_split > 1) {                                                                    \
       hipLaunchKernelGGL((paged_prefill_tiled<T, DD, rt, occ, true, PAD, DL>), grid, block, 0,   \
                          s, a, a.cu_q, a.cu_k, a.table, qtiles, n_split, part);                  \
       hipLaunchKernelGGL((paged_prefill_merge<T, DD>),                                           \

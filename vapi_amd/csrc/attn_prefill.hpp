@@ -61,4 +61,208 @@ __device__ __forceinline__ uint32_t lds_addr(const uint16_t* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint16_t*)p;
 }
 
+// ---- balanced ranges of a prefill launch ------------------------------------
+//
+// A launch whose query tiles do not fill the GPU's workgroup slots evenly
+// (fewer tiles than slots, or a last round that is nearly empty, or tiles of
+// very different lengths) is cut into ranges of equal work instead, one
+// workgroup each: a range may start and end inside a tile and cover whole
+// tiles between. The tiles' order is kv head, then list order, then each
+// sequence from its last tile to its first; XCD x runs a contiguous eighth of
+// the ranges, so the tiles that run together on an XCD share a kv head's K/V.
+// A tile's work is counted in sixteenths of a 32-key step and falls by a
+// constant from a sequence's last tile to its first (the causal mask; not at
+// all with a window), so sums over tiles have a closed form; a piece's share
+// of that count is then its share of the tile's real steps.
+//
+// The first piece of range r that is not a whole tile goes to partial slot
+// 2 r if it starts the range, else to 2 r + 1. The range that starts a tile
+// without ending it describes the tile (PfSplitTile), and the merge joins its
+// piece with the following ranges' first pieces.
+constexpr uint32_t kPfMinSteps = 8;  // per range, in launches of few steps
+
+struct PfSplitTile {
+  uint32_t valid, seq, qt, kh;
+  uint32_t first_slot, last;  // partial slot of the first piece, the last range
+  uint32_t pad[2];
+};
+
+// The plan, in LDS: one entry per sequence of the list (at most kPfSortSeqs,
+// one per lane while it is made). Every wave makes the same one and reads its
+// own, so no barrier stands between.
+struct PfEntry {
+  uint32_t seq, q0, len_q, len_k;
+  uint32_t nt, c_last, fall;  // tiles, the last tile's count, what each earlier one has less
+  uint32_t pad;
+};
+
+// The step of `steps` at count u of c: 0 at 0, all of them at c, never falling
+// between, the same wherever it is computed.
+__device__ __forceinline__ uint32_t pf_step_at(uint32_t u, uint32_t c, uint32_t steps) {
+  return u >= c ? steps : min(steps, (uint32_t)((float)u * ((float)steps / (float)c)));
+}
+
+__device__ __forceinline__ uint32_t pf_tiles_sum(uint32_t c, uint32_t f, uint32_t n) {
+  return n * c - f * (n * (n - 1) / 2);
+}
+
+// A walk over the plan's tiles: tile m from the last of list entry li's.
+struct PfWalk {
+  PfEntry* plan;   // this wave's
+  PfEntry mine;    // this lane's entry, until the first tile is found
+  uint32_t sum;    // and the count of its tiles
+  uint64_t some;   // entries with tiles
+  uint32_t total;  // counts of one kv head
+  uint32_t li, m, kh, c, f, n;  // (uniform) c: the count of the entry's last tile
+  uint32_t seq, q0, len_q, len_k;
+
+  __device__ __forceinline__ void init(const AttnArgs& a, const uint32_t* __restrict__ cu_q,
+                                       const uint32_t* __restrict__ cu_k, uint32_t qtiles,
+                                       uint32_t rows, PfEntry* entries) {
+    const uint32_t lane = threadIdx.x & 63;
+    PfEntry e{0, 0, 0, 0, 0, 16, 0, 0};
+    if (lane < a.pf_seqs_n) {
+      e.seq = a.pf_seqs ? a.pf_seqs[lane] : lane;
+      if (e.seq < a.batch) {
+        e.q0 = cu_q[e.seq], e.len_q = cu_q[e.seq + 1] - e.q0;
+        e.len_k = cu_k[e.seq + 1] - cu_k[e.seq];
+        if (e.len_q >= a.pf_min_q && e.len_q > 0)
+          e.nt = min((uint32_t)(((uint64_t)e.len_q * a.group + rows - 1) / rows), qtiles);
+      }
+    }
+    if (e.nt) {
+      // Steps of the last tile, from its first row's window to its last key.
+      const int32_t offset = (int32_t)(e.len_k - e.len_q);
+      int32_t klo, khi, unused;
+      key_range(offset + (int32_t)((e.nt - 1) * rows / a.group), (int32_t)e.len_k, a.wl, a.wr,
+                klo, unused);
+      key_range(offset + (int32_t)e.len_q - 1, (int32_t)e.len_k, a.wl, a.wr, unused, khi);
+      e.c_last = 16u * (khi >= klo ? (uint32_t)((khi >> 5) - (klo >> 5) + 1) : 1u);
+      if (a.wl < 0 && a.wr >= 0 && e.nt > 1)
+        e.fall = min(rows / (2 * a.group), (e.c_last - 16) / (e.nt - 1));
+    }
+    mine = e;
+    sum = pf_tiles_sum(e.c_last, e.fall, e.nt);
+    some = __ballot(e.nt > 0);
+    total = 0;
+    for (uint64_t left = some; left; left &= left - 1)
+      total += __builtin_amdgcn_readlane(sum, (uint32_t)__builtin_ctzll(left));
+    plan = entries + 64 * (threadIdx.x >> 6);
+    plan[lane] = e;  // for the pieces after the first
+  }
+  // To the tile holding count `at` of kv head kh_, as the walk's first (from
+  // the lanes); returns its place in it.
+  __device__ __forceinline__ uint32_t seek(uint32_t kh_, uint32_t at) {
+    kh = kh_;
+    uint64_t left = some;
+    while (true) {
+      li = (uint32_t)__builtin_ctzll(left);
+      const uint32_t all = __builtin_amdgcn_readlane(sum, li);
+      left &= left - 1;
+      if (at < all || !left) break;
+      at -= all;
+    }
+    c = __builtin_amdgcn_readlane(mine.c_last, li);
+    f = __builtin_amdgcn_readlane(mine.fall, li);
+    n = __builtin_amdgcn_readlane(mine.nt, li);
+    uint32_t hi = n;
+    m = 0;  // pf_tiles_sum(m) <= at < pf_tiles_sum(hi)
+    while (hi - m > 1) {
+      const uint32_t mid = (m + hi) >> 1;
+      if (pf_tiles_sum(c, f, mid) <= at) m = mid;
+      else hi = mid;
+    }
+    seq = __builtin_amdgcn_readlane(mine.seq, li);
+    q0 = __builtin_amdgcn_readlane(mine.q0, li);
+    len_q = __builtin_amdgcn_readlane(mine.len_q, li);
+    len_k = __builtin_amdgcn_readlane(mine.len_k, li);
+    return at - pf_tiles_sum(c, f, m);
+  }
+  __device__ __forceinline__ uint32_t count() const { return c - f * m; }
+  __device__ __forceinline__ void next() {
+    if (++m < n) return;
+    m = 0;
+    const uint64_t after = li < 63 ? some & (~0ull << (li + 1)) : 0ull;
+    if (!after) ++kh;
+    li = (uint32_t)__builtin_ctzll(after ? after : some);
+    const PfEntry e = plan[li];
+    c = __builtin_amdgcn_readfirstlane(e.c_last);
+    f = __builtin_amdgcn_readfirstlane(e.fall);
+    n = __builtin_amdgcn_readfirstlane(e.nt);
+    seq = __builtin_amdgcn_readfirstlane(e.seq);
+    q0 = __builtin_amdgcn_readfirstlane(e.q0);
+    len_q = __builtin_amdgcn_readfirstlane(e.len_q);
+    len_k = __builtin_amdgcn_readfirstlane(e.len_k);
+  }
+  __device__ __forceinline__ PfItem item() const {
+    return PfItem{li, seq, n - 1 - m, kh, q0, len_q, (int32_t)len_k};
+  }
+};
+
+// Workgroup `bid`'s range of at most `ranges`: piece(item, u0, u1, c, slot)
+// for each of its pieces, counts [u0, u1) of the tile's c (slot: its partial,
+// or ~0u for a whole tile), the workgroup's LDS free again between them.
+template <int W, typename Piece>
+__device__ __forceinline__ void pf_walk_range(const AttnArgs& a, const uint32_t* __restrict__ cu_q,
+                                              const uint32_t* __restrict__ cu_k, uint32_t qtiles,
+                                              uint32_t rows, uint32_t ranges,
+                                              PfSplitTile* __restrict__ tiles, uint32_t bid,
+                                              Piece piece) {
+  __shared__ PfEntry entries[64 * W];
+  PfWalk w;
+  w.init(a, cu_q, cu_k, qtiles, rows, entries);
+  // 32-bit counts: the host takes ranges only where S * ranges fits (lengths
+  // past its max_seqlen_k may wrap it: the walk then ends at the last head).
+  const uint32_t S = w.total * a.kvh;
+  const uint32_t nr = min(ranges, (S + 16 * kPfMinSteps - 1) / (16 * kPfMinSteps));
+  if (bid >= nr || !w.some) {
+    if (threadIdx.x == 0) tiles[bid].valid = 0;
+    return;
+  }
+  const uint32_t x = bid % 8, r = x * (nr / 8) + min(x, nr % 8) + bid / 8;
+  uint32_t at = S * r / nr;
+  const uint32_t end = S * (r + 1) / nr;
+  const uint32_t kh0 = at / w.total;
+  uint32_t u0 = w.seek(kh0, at - kh0 * w.total);
+  uint32_t slot = 2 * r, goes_on = 0;
+  while (at < end && w.kh < a.kvh) {
+    const uint32_t c = w.count(), u1 = min(c, u0 + (end - at));
+    const PfItem it = w.item();
+    piece(it, u0, u1, c, u0 == 0 && u1 == c ? ~0u : slot);
+    if (u0 == 0 && u1 < c) {  // starts here, ends in a later range
+      goes_on = 1;
+      if (threadIdx.x == 0) {
+        PfSplitTile t;
+        t.valid = 1, t.seq = it.seq, t.qt = it.qt, t.kh = it.kh, t.first_slot = slot;
+        t.last = min(((at + c) * nr + S - 1) / S, nr) - 1;
+        t.pad[0] = t.pad[1] = 0;
+        tiles[r] = t;
+      }
+    }
+    at += u1 - u0;
+    if (at >= end) break;
+    u0 = 0, slot = 2 * r + 1;
+    w.next();
+    __syncthreads();
+  }
+  if (threadIdx.x == 0 && !goes_on) tiles[r].valid = 0;
+}
+
+// The launch's side of it: at most one range per CU; the split tiles lead the
+// workspace, the partials follow.
+constexpr uint32_t kPfMaxRanges = 256;
+constexpr uint64_t kPfMaxCount = 0xFFFFFFFFull / kPfMaxRanges;  // of all tiles
+constexpr size_t kPfRangeHead = kPfMaxRanges * sizeof(PfSplitTile);
+struct PfRangePlan {
+  uint32_t ranges;  // 0: none, the launch runs its tiles as they are
+  size_t bytes;     // of workspace
+};
+// For `items` tiles if every sequence is as long as the longest, of at most
+// max_k keys and max_q queries, which would otherwise run as n_split shares each, `slots` at
+// once, step_us a step; partials of part_bytes each.
+PfRangePlan pf_range_plan(uint64_t items, uint32_t max_q, uint32_t max_k, uint32_t slots,
+                          uint32_t n_split, float step_us, uint64_t part_bytes, size_t ws_bytes);
+void launch_prefill_range_merge(const AttnArgs& a, uint32_t ranges, uint32_t rows, uint32_t dtype,
+                                uint32_t head_dim, const void* ws, hipStream_t s);
+
 }  // namespace vk

@@ -258,17 +258,13 @@ __device__ __forceinline__ void f32_rows(const AttnArgs& a, const uint32_t* __re
   }
 }
 
-// kSplit: the keys a workgroup would walk are cut into n_split contiguous
-// runs of steps, one workgroup each (a batch too small to fill the GPU with
-// query tiles alone); each writes its rows' (m, l, o / l) to `part` for the
-// merge. DL: the 16-column d tiles that hold head_dim (kPad; D / 16
-// otherwise): the MFMAs and reads of the tiles past them are left out.
-template <int D, int RT, bool kSplit, bool kPad, int DL = D / 16>
-__global__ __launch_bounds__(kPf32Threads, 1) void paged_prefill_f32x3(
-    AttnArgs a, const uint32_t* __restrict__ cu_q, const uint32_t* __restrict__ cu_k,
-    const uint32_t* __restrict__ table, uint32_t qtiles, uint32_t n_split_arg,
-    float* __restrict__ part) {
-  const uint32_t n_split = kSplit ? n_split_arg : 1u;
+// One item: query tile it.qt of a sequence and kv head. kSplit, u0, u1, c,
+// pb: as prefill_piece's. DL: the 16-column d tiles that hold head_dim (kPad;
+// D / 16 otherwise): the MFMAs and reads of the tiles past them are left out.
+template <int D, int RT, int kSplit, bool kPad, int DL>
+__device__ __forceinline__ void x3_piece(const AttnArgs& a, const uint32_t* __restrict__ table,
+                                         const PfItem& it, uint32_t u0, uint32_t u1, uint32_t c_all,
+                                         char* pb) {
   constexpr uint32_t kPf32Rows = x3_rows(RT);
   constexpr int DT = D / 16, KCL = (DL + 1) / 2;
   constexpr uint32_t kPlane = 32 * D;       // elements of one plane of one tensor
@@ -277,12 +273,7 @@ __global__ __launch_bounds__(kPf32Threads, 1) void paged_prefill_f32x3(
   constexpr int kPlaneB = kPlane * 2;
   __shared__ __attribute__((aligned(16))) uint16_t kpl[2][3 * kPlane], vpl[2][3 * kPlane];
   __shared__ uint4 raw[kUnits][2][kPf32Threads];
-  __shared__ uint32_t order[64 * kPf32Waves];
-  const uint32_t hr = blockIdx.x / a.kvh, split = hr % n_split;
-  PfItem it;
-  if (!prefill_item<kPf32Waves>(a, cu_q, cu_k, (hr / n_split) * a.kvh + blockIdx.x % a.kvh, qtiles,
-                                kPf32Rows, order, it))
-    return;
+  __shared__ uint32_t notes_lds;
   const uint32_t qt = it.qt, kh = it.kh, q0 = it.q0;
   const uint32_t G = a.group, nrows = it.len_q * G;
   const uint32_t row_base = qt * kPf32Rows;
@@ -301,7 +292,7 @@ __global__ __launch_bounds__(kPf32Threads, 1) void paged_prefill_f32x3(
   if (kSplit) {
     const int32_t first = klo & ~31;
     const uint32_t steps = khi >= klo ? (uint32_t)(((khi & ~31) - first) / 32 + 1) : 0u;
-    const uint32_t a0 = split * steps / n_split, a1 = (split + 1) * steps / n_split;
+    const uint32_t a0 = pf_step_at(u0, c_all, steps), a1 = pf_step_at(u1, c_all, steps);
     klo = max(klo, first + 32 * (int32_t)a0);
     khi = min(khi, first + 32 * (int32_t)a1 - 1);
   }
@@ -522,22 +513,19 @@ __global__ __launch_bounds__(kPf32Threads, 1) void paged_prefill_f32x3(
   wait_vmcnt<0>();  // no load may land in LDS after the workgroup ends
 
   // Values without a split anywhere in the workgroup's share: f32 MFMAs.
-  char* const pb = kSplit ? (char*)part + ((uint64_t)((it.li * a.kvh + kh) * qtiles + qt) * n_split +
-                                           split) * pf_part_bytes(kPf32Rows, D)
-                          : nullptr;
-  if (tid == 0) order[0] = 0;
+  if (tid == 0) notes_lds = 0;
   __syncthreads();
   {
     const uint32_t notes =
         magnitude_notes(mag_q) | magnitude_notes(mag_k) << 3 | magnitude_notes(mag_v) << 6;
-    if (lane == 0) atomicOr(&order[0], notes);
+    if (lane == 0) atomicOr(&notes_lds, notes);
   }
   __syncthreads();
-  if (needs_f32(__builtin_amdgcn_readfirstlane(order[0]))) {
+  if (needs_f32(__builtin_amdgcn_readfirstlane(notes_lds))) {
 #pragma unroll 1
     for (uint32_t t = 0; t < (uint32_t)RT; ++t)
-      f32_rows<D, 1, kPad, D / 16, false>(a, tab, kh, q0, nrows, row0 + 16 * t, offset, len_k, klo, khi,
-                                   pb, wrow0 + 16 * t, kPf32Rows);
+      f32_rows<D, 1, kPad, D / 16, false>(a, tab, kh, q0, nrows, row0 + 16 * t, offset, len_k, klo,
+                                          khi, kSplit ? pb : nullptr, wrow0 + 16 * t, kPf32Rows);
     return;
   }
 #pragma unroll
@@ -546,7 +534,8 @@ __global__ __launch_bounds__(kPf32Threads, 1) void paged_prefill_f32x3(
     const float inv = lt > 0.f ? 1.f / lt : 0.f;
     const uint32_t r = row0 + 16 * t + col;
     float* dst;
-    if constexpr (kSplit) {
+    const bool partial = kSplit == 1 || (kSplit == 2 && pb);
+    if (partial) {
       const uint32_t pr = wrow0 + 16 * t + col;
       if (g == 0) *(float2*)(pb + (uint64_t)pr * 8) = make_float2(m_run[t], lt);
       dst = (float*)(pb + (uint64_t)kPf32Rows * 8) + (uint64_t)pr * D;
@@ -557,11 +546,51 @@ __global__ __launch_bounds__(kPf32Threads, 1) void paged_prefill_f32x3(
     }
 #pragma unroll
     for (int k = 0; k < DL; ++k)
-      if (!kPad || kSplit || 16 * k + 4 * g < a.hd)
+      if (!kPad || partial || 16 * k + 4 * g < a.hd)
         *(float4*)(dst + 16 * k + 4 * g) = make_float4(o[t][k][0] * inv, o[t][k][1] * inv,
                                                        o[t][k][2] * inv, o[t][k][3] * inv);
   }
 }
+// Workgroups of a launch: an item each, or (kSplit) one of n_split equal
+// shares of each item's steps, to be merged (a batch too small to fill the
+// GPU with query tiles alone).
+template <int D, int RT, bool kSplit, bool kPad, int DL = D / 16>
+__global__ __launch_bounds__(kPf32Threads, 1) void paged_prefill_f32x3(
+    AttnArgs a, const uint32_t* __restrict__ cu_q, const uint32_t* __restrict__ cu_k,
+    const uint32_t* __restrict__ table, uint32_t qtiles, uint32_t n_split_arg,
+    float* __restrict__ part) {
+  constexpr uint32_t kRows = x3_rows(RT);
+  const uint32_t n_split = kSplit ? n_split_arg : 1u;
+  __shared__ uint32_t order[64 * kPf32Waves];
+  const uint32_t hr = blockIdx.x / a.kvh, split = hr % n_split;
+  PfItem it;
+  if (!prefill_item<kPf32Waves>(a, cu_q, cu_k, (hr / n_split) * a.kvh + blockIdx.x % a.kvh, qtiles,
+                                kRows, order, it))
+    return;
+  char* pb = nullptr;
+  if (kSplit)
+    pb = (char*)part + ((uint64_t)((it.li * a.kvh + it.kh) * qtiles + it.qt) * n_split + split) *
+                           pf_part_bytes(kRows, D);
+  x3_piece<D, RT, kSplit ? 1 : 0, kPad, DL>(a, table, it, split, split + 1, n_split, pb);
+}
+
+// The same over ranges of equal work (see attn_prefill.hpp).
+template <int D, int RT, bool kPad, int DL = D / 16>
+__global__ __launch_bounds__(kPf32Threads, 1) void paged_prefill_f32x3_ranges(
+    AttnArgs a, const uint32_t* __restrict__ cu_q, const uint32_t* __restrict__ cu_k,
+    const uint32_t* __restrict__ table, uint32_t qtiles, uint32_t ranges,
+    PfSplitTile* __restrict__ tiles, char* __restrict__ part) {
+  constexpr uint32_t kRows = x3_rows(RT);
+  pf_walk_range<kPf32Waves>(a, cu_q, cu_k, qtiles, kRows, ranges, tiles, blockIdx.x,
+                            [&](const PfItem& it, uint32_t u0, uint32_t u1, uint32_t c,
+                                uint32_t slot) __attribute__((always_inline)) {
+                              x3_piece<D, RT, 2, kPad, DL>(
+                                  a, table, it, u0, u1, c,
+                                  slot == ~0u ? nullptr
+                                              : part + (uint64_t)slot * pf_part_bytes(kRows, D));
+                            });
+}
+
 // kSplit: the keys a wave would walk are cut into n_split contiguous runs
 // of steps, one wave each (a batch too small to fill the GPU with query
 // tiles alone); each writes its rows' (m, l, o / l) to `part`
@@ -616,6 +645,7 @@ __global__ __launch_bounds__(64 * kPfF32Waves, 1) void paged_prefill_f32(
 
 
 constexpr int kPfF32RowTiles = 2;
+constexpr float kX3StepUs = 2.82f;  // a workgroup's 32-key step with one row tile per wave
 
 // The kernel of a launch of n_seqs sequences: rows per item and the items
 // that fill a 256-CU GPU.
@@ -652,6 +682,21 @@ static F32Plan f32_plan(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t 
   return p;
 }
 
+// The same launch in ranges: one row tile per wave (with two, the walk over a
+// range's pieces does not fit the registers beside the kernel's).
+static F32Plan f32_range_plan(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_q) {
+  F32Plan p = f32_plan(n_seqs, kvh, group, max_q);
+  const uint64_t all = (uint64_t)max_q * group;
+  // (Ranges balance the items that few rows would leave half idle: 40
+  // sequences, 8 kv heads, 64 rows over ~1,000 keys: 378 us with f32 MFMAs.)
+  p.x3 = p.x3 || all > 32;
+  p.row_tiles = 1;
+  p.rows = x3_rows(1);
+  p.qtiles = (uint32_t)((all + p.rows - 1) / p.rows);
+  p.items = (uint64_t)p.qtiles * kvh * n_seqs;
+  return p;
+}
+
 uint64_t prefill_f32_items(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_q) {
   return f32_plan(n_seqs, kvh, group, max_q).items;
 }
@@ -669,33 +714,53 @@ static uint32_t pf32_splits(const F32Plan& p, uint32_t max_k, uint32_t head_dim,
   return (uint32_t)n;
 }
 
+static PfRangePlan f32_ranges(const F32Plan& p, uint32_t n_seqs, uint32_t max_q, uint32_t max_k,
+                              uint32_t head_dim, uint64_t bytes) {
+  if (!p.x3 || n_seqs > kPfSortSeqs) return PfRangePlan{0, 0};
+  return pf_range_plan(p.items, max_q, max_k, 256, pf32_splits(p, max_k, head_dim, bytes),
+                       kX3StepUs, pf_part_bytes(p.rows, head_dim), bytes);
+}
+
 size_t prefill_f32_split_bytes(uint32_t batch, uint32_t kvh, uint32_t group, uint32_t head_dim,
                                uint32_t max_q, uint32_t max_k) {
   if (max_q <= 1) return 0;
   const F32Plan p = f32_plan(batch, kvh, group, max_q);
   const uint32_t n = pf32_splits(p, max_k, head_dim, ~0ull);
-  return n > 1 ? (size_t)(p.items * n * pf_part_bytes(p.rows, head_dim)) : 0;
+  const size_t split = n > 1 ? (size_t)(p.items * n * pf_part_bytes(p.rows, head_dim)) : 0;
+  const F32Plan r = f32_range_plan(batch, kvh, group, max_q);
+  return std::max(split, f32_ranges(r, batch, max_q, max_k, head_dim, ~0ull).bytes);
 }
 
 void launch_prefill_f32(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, uint32_t head_dim,
                         void* split_ws, size_t split_ws_bytes, hipStream_t s) {
   AttnArgs a = a_in;
-  const F32Plan p = f32_plan(a.pf_seqs_n, a.kvh, a.group, max_q);
-  const uint32_t qtiles = p.qtiles;
-  a.pf_sort = prefill_sorts(a.pf_seqs_n, qtiles);
   // No split without a workspace, nor for a deterministic call (its output
   // must not depend on the workspace it is given).
+  const bool split_ok = split_ws && !a.deterministic;
+  F32Plan p = f32_range_plan(a.pf_seqs_n, a.kvh, a.group, max_q);
+  const PfRangePlan rp = split_ok ? f32_ranges(p, a.pf_seqs_n, max_q, max_k, head_dim, split_ws_bytes)
+                                  : PfRangePlan{0, 0};
+  if (!rp.ranges) p = f32_plan(a.pf_seqs_n, a.kvh, a.group, max_q);
+  const uint32_t qtiles = p.qtiles;
+  a.pf_sort = prefill_sorts(a.pf_seqs_n, qtiles);
   const uint32_t n_split =
-      split_ws && !a.deterministic ? pf32_splits(p, max_k, head_dim, split_ws_bytes) : 1;
+      split_ok && !rp.ranges ? pf32_splits(p, max_k, head_dim, split_ws_bytes) : 1;
   const uint64_t items = p.items * n_split;
   const uint32_t wgs = (uint32_t)((items + kPfF32Waves - 1) / kPfF32Waves);
   float* part = n_split > 1 ? (float*)split_ws : nullptr;
 #define VK_X3(DD, RT, SPLIT, PAD, CL)                                                            \
   hipLaunchKernelGGL((paged_prefill_f32x3<DD, RT, SPLIT, PAD, CL>), dim3((uint32_t)items),       \
                      dim3(kPf32Threads), 0, s, a, a.cu_q, a.cu_k, a.table, qtiles, n_split, part)
+#define VK_X3R(DD, PAD, CL)                                                                      \
+  hipLaunchKernelGGL((paged_prefill_f32x3_ranges<DD, 1, PAD, CL>), dim3(rp.ranges),              \
+                     dim3(kPf32Threads), 0, s, a, a.cu_q, a.cu_k, a.table, qtiles, rp.ranges,    \
+                     (PfSplitTile*)split_ws, (char*)split_ws + kPfRangeHead)
 #define VK_PF32(DD, PAD, CL)                                                                     \
   do {                                                                                           \
-    if (p.x3) {                                                                                  \
+    if (rp.ranges) {                                                                             \
+      VK_X3R(DD, PAD, CL);                                                                       \
+      launch_prefill_range_merge(a, rp.ranges, p.rows, VAPI_KV_F32, DD, split_ws, s);            \
+    } else if (p.x3) {                                                                                  \
       if (p.row_tiles == 2) {                                                                    \
         VK_X3(DD, 2, false, PAD, CL); /* enough items: never split */                            \
       } else if (n_split > 1) {                                                                  \
@@ -729,6 +794,7 @@ void launch_prefill_f32(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, ui
     else VK_PF32(64, true, 4);
   }
 #undef VK_PF32
+#undef VK_X3R
 #undef VK_X3
 }
 
