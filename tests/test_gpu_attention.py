@@ -712,11 +712,15 @@ def test_small_prefill_batches_split_their_keys_and_match_the_oracle(case):
 
 ORDER_CASES = [
     # dtype, heads, kvh, d, n_seqs: tiles of 256 rows (128 at head_dim 256)
-    (torch.bfloat16, 4, 1, 64, 2),     # two sequences: the smallest sorted list
+    (torch.bfloat16, 4, 1, 64, 2),     # two sequences
     (torch.float16, 21, 3, 128, 9),    # kv heads that do not divide the XCDs
     (torch.bfloat16, 32, 8, 128, 64),  # one sequence per lane
     (torch.bfloat16, 16, 2, 64, 65),   # past the sort: list order
     (torch.bfloat16, 8, 2, 256, 5),
+    # More items than CUs, so sorted (few items keep list order):
+    (torch.bfloat16, 64, 64, 64, 2),
+    (torch.float16, 21, 3, 128, 40),
+    (torch.bfloat16, 32, 8, 256, 12),
 ]
 
 

@@ -126,13 +126,17 @@ struct PfItem {
 // equal sequences 1,065 -> 1,057 us. Launches of one tile per sequence and
 // of more sequences than lanes keep list order, which needs no walk over
 // the list (64 sequences of 32 fresh tokens: 16.8 us, 18.2 sorted; 17.4
-// before).
+// before). So do launches of at most a workgroup per CU, where all items
+// start at once and their order changes nothing: 6 x 100-200 fresh tokens
+// at head_dim 64 (96 items) take 10.8 us, 11.3 sorted, 3 x 100-200 of 28 q /
+// 4 kv heads at head_dim 96 12.2, 12.5 sorted.
 // Each of the workgroup's W waves holds one sequence per lane and counts the
 // tiles before it among its share of the others; `tmp` (W x 64 words of LDS)
 // adds the shares up. Every thread of the workgroup calls this.
 constexpr uint32_t kPfSortSeqs = 64;
-inline bool prefill_sorts(uint32_t n_seqs, uint32_t qtiles) {
-  return n_seqs > 1 && n_seqs <= kPfSortSeqs && qtiles > 1;
+constexpr uint32_t kPfSortItems = 256;  // one per CU
+inline bool prefill_sorts(uint32_t n_seqs, uint32_t qtiles, uint64_t items) {
+  return n_seqs > 1 && n_seqs <= kPfSortSeqs && qtiles > 1 && items > kPfSortItems;
 }
 template <int W>
 __device__ __forceinline__ bool prefill_item(const AttnArgs& a, const uint32_t* __restrict__ cu_q,

@@ -712,7 +712,6 @@ void launch_mixed(const AttnArgs& a_in, void* workspace, uint32_t max_q, uint32_
   decode_bind(c, workspace, head_dim);
   const uint32_t nwg = c.num_waves / kDecodeWavesPerWG;
   const uint32_t qtiles = (uint32_t)(((uint64_t)max_q * c.group + kMixRows - 1) / kMixRows);
-  c.pf_sort = prefill_sorts(c.pf_seqs_n, qtiles);
   const uint64_t base = (uint64_t)qtiles * c.kvh * c.pf_seqs_n;
   // The prefill workgroups run beside the decode's, one per CU: as many key
   // splits as keep them within one round of the GPU's CUs (a second round
@@ -727,6 +726,7 @@ void launch_mixed(const AttnArgs& a_in, void* workspace, uint32_t max_q, uint32_
                               std::min<uint64_t>(split_ws_bytes, kPfSplitMaxBytes))
       --n_split;
   }
+  c.pf_sort = prefill_sorts(c.pf_seqs_n, qtiles, base * n_split);
   float* part = n_split > 1 ? (float*)split_ws : nullptr;
   const dim3 grid((uint32_t)(nwg + base * n_split)), block(256);
   const size_t lds = (c.batch + 1) * sizeof(uint32_t);
@@ -803,7 +803,6 @@ void launch_prefill(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, uint32
   AttnArgs a = a_in;
   const uint32_t rows = pf_rows(head_dim);
   const uint32_t qtiles = (uint32_t)(((uint64_t)max_q * a.group + rows - 1) / rows);
-  a.pf_sort = prefill_sorts(a.pf_seqs_n, qtiles);
   const uint64_t base = (uint64_t)qtiles * a.kvh * a.pf_seqs_n;
   // As many splits as the workspace given holds (none without one); a
   // deterministic call does not split, so its output does not depend on
@@ -816,6 +815,7 @@ void launch_prefill(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, uint32
           ? pf_range_plan(base, max_q, max_k, pf_slots(head_dim), n_split, kPfStepUs,
                           pf_part_bytes(rows, head_dim), split_ws_bytes)
           : PfRangePlan{0, 0};
+  a.pf_sort = prefill_sorts(a.pf_seqs_n, qtiles, base * n_split);
   float* part = n_split > 1 ? (float*)split_ws : nullptr;
   const dim3 grid((uint32_t)(base * n_split)), block(kPfThreads);
 #define VK_PF(T, DD, PAD, DL)                                                                    \

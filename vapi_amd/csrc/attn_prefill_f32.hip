@@ -742,10 +742,10 @@ void launch_prefill_f32(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, ui
                                   : PfRangePlan{0, 0};
   if (!rp.ranges) p = f32_plan(a.pf_seqs_n, a.kvh, a.group, max_q);
   const uint32_t qtiles = p.qtiles;
-  a.pf_sort = prefill_sorts(a.pf_seqs_n, qtiles);
   const uint32_t n_split =
       split_ok && !rp.ranges ? pf32_splits(p, max_k, head_dim, split_ws_bytes) : 1;
   const uint64_t items = p.items * n_split;
+  a.pf_sort = prefill_sorts(a.pf_seqs_n, qtiles, items);
   const uint32_t wgs = (uint32_t)((items + kPfF32Waves - 1) / kPfF32Waves);
   float* part = n_split > 1 ? (float*)split_ws : nullptr;
 #define VK_X3(DD, RT, SPLIT, PAD, CL)                                                            \
