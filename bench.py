@@ -258,7 +258,7 @@ def bench_fused_step(d, steps, warmup):
             "two_calls_graph_us": round(g_two * 1e3, 2), "fused_graph_us": round(g_fused * 1e3, 2)}
 
 
-# ---- the VALU kernel (f32 pools, other head dims) ---------------------------------
+# ---- f32 pools, other head dims ---------------------------------
 
 def bench_mixed_step(d, steps, warmup):
     """A chunked-prefill serving step on config 2's pool: its first 63
@@ -308,10 +308,10 @@ def bench_mixed_step(d, steps, warmup):
 
 def bench_valu(steps, warmup):
     """f32 pools: config 0 (Qwen3-0.6B-shaped f32 decode, the reference's CPU
-    parity case: at most 512 keys, so the VALU kernel in one launch), config
+    parity case: at most 512 keys, so the short-context kernel), config
     2's batch over an f32 pool (1.5 GB of K/V, the f32-MFMA decode stream),
     the same batch at head_dim 80 (the stream padded to 128), and config 3
-    on an f32 pool (the f32-MFMA prefill) at head_dim 128 and 80."""
+    on an f32 pool (the bf16-split prefill) at head_dim 128 and 80."""
     out = {}
     for name, w, heads, kvh, d in (("cfg0_f32", workload.config0_decode_small(), 16, 8, None),
                                    ("cfg2_shape_f32", workload.config2_decode(), 32, 8, None),
@@ -331,7 +331,7 @@ def bench_valu(steps, warmup):
         kv = int(w.lens.sum()) * 2 * kvh * d * 4
         out[name] = dict(us=ms * 1e3, graph_us=gms * 1e3, kv_bytes=kv,
                          gbs=kv / (ms * 1e-3) / 1e9, graph_gbs=kv / (gms * 1e-3) / 1e9,
-                         path=("VALU kernel" if name == "cfg0_f32"
+                         path=("short-context decode" if name == "cfg0_f32"
                                else "f32 MFMA decode stream (head_dim 80: padded to 128)"
                                if name.endswith("d80") else "f32 MFMA decode stream"))
         log(f"f32 attention {name}: {ms * 1e3:.1f} us ({gms * 1e3:.1f} us in a graph), "

@@ -225,9 +225,9 @@ int vapi_kv_gather(const vapi_kv_pool* pool, uint32_t layer,
  *   64 or 128, or another multiple of 4 below 128 run at the next of them,
  *   runs the decode stream and an f32 prefill kernel, sized the
  *   same way (the f32 prefill's key split is the optional part; a
- *   pure-decode f32 call over at
- *   most 512 keys per sequence and 8,192 in all runs the VALU kernel). On
- *   the VALU path (those small calls, other head dims, groups of more than 256
+ *   pure-decode f32 call over at most 512 keys per sequence and 8,192 in
+ *   all runs the short-context kernel where that takes it, else the VALU
+ *   kernel, whose size it gets). On the VALU path (other head dims, groups of more than 256
  *   query heads per kv head, block sizes below 16) it holds the split-context partials and
  *   grows with the batch, max_seqlen_q and max_seqlen_k (0 while
  *   max_seqlen_k <= 64; small batches split their keys into chunks of 64
