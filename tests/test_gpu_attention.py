@@ -16,6 +16,7 @@ import pytest
 import torch
 
 import oracle
+from prefill_plan import route
 from vapi_amd import _lib, workload
 from vapi_amd.attention import (ForwardBatch, PreparedAttention, paged_attention,
                                 paged_attention_prepared, paged_attention_windowed)
@@ -906,3 +907,34 @@ def test_prefill_in_ranges_of_equal_work_matches_the_oracle(case):
             got = torch.full_like(q, float("nan"))
             paged_attention_prepared(q, c, 0, prep, d ** -0.5, left, out=got)
             assert max_abs(got, want) <= tol
+
+
+@pytest.mark.parametrize("dtype,heads,kvh,n,q_len", [(torch.bfloat16, 32, 8, 15, 128),
+                                                     (torch.float32, 16, 8, 1, 512)])
+def test_ranges_at_the_longest_context_they_are_taken_for(dtype, heads, kvh, n, q_len):
+    """Where the counts of a launch's tiles are the largest, against the same
+    call unsplit: every sequence over one shared table."""
+    f32 = dtype == torch.float32
+    k_len = max(k for k in range(4096, 1 << 20, 31)
+                if route(f32, n, heads, kvh, q_len, k, 128).ranges)
+    nb = -(-k_len // 16)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    c = PagedKvCache(1, nb, 16, kvh, 128, dtype)
+    c.k[0].normal_(generator=g)
+    c.v[0].normal_(generator=g)
+    q = torch.randn((n * q_len, heads, 128), generator=g, device=DEV, dtype=torch.float32).to(dtype)
+    table = np.random.default_rng(5).permutation(nb).tolist()
+    batch = ForwardBatch(cu_seqlens_q=[q_len * i for i in range(n + 1)],
+                         cu_seqlens_k=[k_len * i for i in range(n + 1)],
+                         block_tables=[table] * n, max_seqlen_q=q_len, max_seqlen_k=k_len)
+    out = {}
+    for det in (False, True):  # deterministic: no ranges
+        prep = PreparedAttention.from_batch(batch, DEV, cache=c, num_heads=heads,
+                                            deterministic=det)
+        got = torch.full_like(q, float("nan"))
+        out[det] = paged_attention_prepared(q, c, 0, prep, 128 ** -0.5, out=got)
+    assert bool(torch.isfinite(out[True]).all())
+    # Relative, as outputs here are ~1 / sqrt(keys). f32: each call adds up to
+    # k_len / 32 steps, a rounding of 2^-24 each, two sums (o and l) in both.
+    tol = (4 * (k_len / 32) ** 0.5 * 2.0 ** -24 if f32 else 2e-2) * float(out[True].abs().max())
+    assert max_abs(out[False], out[True]) <= tol

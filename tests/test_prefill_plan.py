@@ -1,0 +1,84 @@
+"""The plan of prefill launches that run as ranges of equal work, on the CPU:
+every range walked with the kernel's own arithmetic, each tile's counts
+covered once, each split tile's description naming its pieces."""
+import numpy as np
+import pytest
+
+from prefill_plan import check_walk, route
+
+
+def equal(f32, n, heads, kvh, q, k, d=128):
+    r = route(f32, n, heads, kvh, q, k, d)
+    return r, (check_walk(r, [q] * n, [k] * n, heads, kvh) if r.ranges else 0)
+
+
+# f32, sequences, q heads, kv heads, queries each: shapes whose counts pass
+# 2^24 at long contexts.
+LONG = [
+    (False, 1, 32, 8, 512), (False, 2, 32, 8, 512), (False, 63, 32, 8, 64),
+    (False, 22, 32, 32, 200), (False, 15, 32, 8, 128), (False, 2, 32, 8, 960),
+    (False, 20, 32, 8, 192), (True, 1, 16, 8, 512), (True, 3, 16, 8, 300),
+]
+
+
+@pytest.mark.parametrize("case", LONG, ids=lambda c: f"f32-{c[0]}-n{c[1]}-kvh{c[3]}-q{c[4]}")
+def test_ranges_hold_up_to_the_longest_context_they_are_taken_for(case):
+    """Every context for the last 1,500 keys that ranges are taken for (they
+    end where the counts' products would leave 32 bits), and around the
+    largest that an unbounded product would allow."""
+    f32, n, heads, kvh, q = case
+    lo, hi = 4096, 1 << 20
+    assert not route(f32, n, heads, kvh, q, hi, 128).ranges
+    # The last context, on a grid coarse enough that equal shares taken here
+    # and there below it don't matter.
+    ks = [k for k in range(lo, hi, 997) if route(f32, n, heads, kvh, q, k, 128).ranges]
+    assert ks
+    for k in range(max(ks[-1] - 1500, q), ks[-1] + 2000, 7):
+        r, bad = equal(f32, n, heads, kvh, q, k)
+        assert bad == 0, (k, r)
+    # Ragged: one sequence at that length, the others anywhere below.
+    rng = np.random.default_rng(n)
+    for _ in range(20):
+        k = ks[-1] - int(rng.integers(0, 300))
+        r = route(f32, n, heads, kvh, q, k, 128)
+        lens_q = [int(x) for x in rng.integers(1, q + 1, n)]
+        lens_k = [int(x) for x in rng.integers(q, k + 1, n)]
+        lens_q[0], lens_k[-1] = q, k
+        for wl, wr in ((-1, 0), (-1, -1), (5000, 0)):
+            if r.ranges:
+                assert check_walk(r, lens_q, lens_k, heads, kvh, wl, wr) == 0
+
+
+@pytest.mark.parametrize("f32", [False, True])
+def test_ranges_hold_over_ragged_batches(f32):
+    rng = np.random.default_rng(7 + f32)
+    taken = 0
+    for _ in range(4000):
+        n = int(rng.integers(1, 65))
+        kvh = int(rng.choice([1, 2, 3, 4, 8, 32]))
+        heads = kvh * int(rng.choice([1, 2, 4, 7, 16]))
+        q = int(np.exp(rng.uniform(np.log(2), np.log(3000))))
+        k = q + int(np.exp(rng.uniform(0, np.log(60000))))
+        d = int(rng.choice([64, 128]))
+        ws = (1 << 64) - 1 if rng.random() < 0.5 else int(np.exp(rng.uniform(9, 19)))
+        r = route(f32, n, heads, kvh, q, k, d, True, ws)
+        if not r.ranges:
+            continue
+        taken += 1
+        assert r.range_bytes <= ws
+        lens_q = [int(x) for x in rng.integers(0, q + 1, n)]
+        lens_k = [max(l, int(x)) for l, x in zip(lens_q, rng.integers(0, k + 1, n))]
+        lens_q[-1], lens_k[-1] = q, k
+        wl = -1 if rng.random() < 0.7 else int(rng.integers(0, k))
+        wr = int(rng.choice([-1, 0, 0, 5]))
+        assert check_walk(r, lens_q, lens_k, heads, kvh, wl, wr) == 0, (r, lens_q, lens_k, wl, wr)
+    assert taken > 200
+
+
+def test_lengths_past_the_hosts_bound_stay_within_the_counts():
+    """max_seqlen_k below the real lengths costs balance, not coverage."""
+    for n, q, k in ((3, 512, 8192), (10, 100, 9000), (1, 512, 400000)):
+        r = route(False, n, 32, 8, q, k, 128)
+        assert r.ranges
+        assert check_walk(r, [q] * n, [1 << 24] * n, 32, 8) == 0
+        assert check_walk(r, [q] * n, [k] * (n - 1) + [1 << 30], 32, 8) == 0

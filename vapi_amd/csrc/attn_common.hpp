@@ -26,6 +26,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "prefill_plan.hpp"
 
 namespace vk {
 
@@ -85,12 +86,6 @@ struct AttnArgs {
   uint32_t hd;
 };
 
-__device__ __forceinline__ void key_range(int32_t p, int32_t len_k, int32_t wl,
-                                          int32_t wr, int32_t& lo, int32_t& hi) {
-  lo = wl >= 0 ? max(0, p - wl) : 0;
-  hi = wr >= 0 ? min(len_k - 1, p + wr) : len_k - 1;
-}
-
 // Workgroup -> work item. The hardware deals workgroups round-robin to the
 // 8 XCDs (linear id % 8); each XCD here gets a contiguous range of work
 // items, so the q-tiles of one (sequence, kv head), which read the same K/V,
@@ -133,11 +128,6 @@ struct PfItem {
 // Each of the workgroup's W waves holds one sequence per lane and counts the
 // tiles before it among its share of the others; `tmp` (W x 64 words of LDS)
 // adds the shares up. Every thread of the workgroup calls this.
-constexpr uint32_t kPfSortSeqs = 64;
-constexpr uint32_t kPfSortItems = 256;  // one per CU
-inline bool prefill_sorts(uint32_t n_seqs, uint32_t qtiles, uint64_t items) {
-  return n_seqs > 1 && n_seqs <= kPfSortSeqs && qtiles > 1 && items > kPfSortItems;
-}
 template <int W>
 __device__ __forceinline__ bool prefill_item(const AttnArgs& a, const uint32_t* __restrict__ cu_q,
                                              const uint32_t* __restrict__ cu_k, uint32_t i,
@@ -700,13 +690,6 @@ __device__ __forceinline__ void store_row_f32(float* row, const floatx4 (&o)[D /
         *(float4*)(row + 64 * h + 16 * g + 4 * i) =
           make_float4(o[4 * h][i] * scale, o[4 * h + 1][i] * scale, o[4 * h + 2][i] * scale,
                       o[4 * h + 3][i] * scale);
-}
-
-// Bytes of one (item, split) partial block of a prefill key split: (m, l)
-// f32 per row, then o / l per row in f32 (the split adds no rounding before
-// the merge).
-__host__ __device__ constexpr uint64_t pf_part_bytes(uint32_t rows, uint32_t d) {
-  return (uint64_t)rows * (8 + 4 * d);
 }
 
 // ---- launchers (one per translation unit) ----------------------------------

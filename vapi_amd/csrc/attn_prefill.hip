@@ -23,8 +23,6 @@
 
 namespace vk {
 
-constexpr int kPfWaves = 8;
-constexpr int kPfThreads = 64 * kPfWaves;
 // ---- K and V staged by direct global-to-LDS loads --------------------------
 //
 // Rows keep the pool's order (key rows of D elements); each row's 16-byte
@@ -518,7 +516,7 @@ __global__ __launch_bounds__(256) void paged_prefill_range_merge(
   const uint32_t blocks_per_item = rows_per_item / (256 / (D / 4));
   const uint32_t r = blockIdx.x / blocks_per_item;
   const PfSplitTile t = tiles[r];
-  if (!t.valid) return;
+  if (!t.valid || t.last >= gridDim.x / blocks_per_item) return;
   const uint64_t stride = pf_part_bytes(rows_per_item, D);
   prefill_merge_rows<T, D>(a, t.seq, t.qt, t.kh, rows_per_item, blockIdx.x % blocks_per_item,
                            t.last - r + 1, [&](uint32_t s) {
@@ -534,106 +532,11 @@ __global__ __launch_bounds__(256) void paged_prefill_merge(AttnArgs a, uint32_t 
   prefill_merge_body<T, D>(a, qtiles, rows_per_item, n_split, part, blockIdx.x);
 }
 
-// Row tiles (16 rows each) per wave, and workgroups per CU at head_dim 128.
-// At head_dim 256 a wave holds one row tile (its O and Q^T fragments, 64 +
-// 32 registers, beside a 64-register K tile: two tiles would not fit the
-// 256 registers of a wave at two waves per SIMD), and the ring's six
-// buffers take 96 KiB of LDS.
-constexpr int kPfRowTiles = 2;
-constexpr int kPfRowTiles256 = 1;
-constexpr int kPfOcc = 1;
-// head_dim 64 fits in 128 registers: two workgroups per CU (four waves per
-// SIMD) measured 1% faster than one on a config-3-shaped batch (676-678
-// against 669-673 TFLOP/s), and four row tiles per wave at one workgroup
-// per CU no faster (817-819 against 823-824).
-constexpr int kPfOcc64 = 2;
-
-// Query rows of one prefill workgroup.
-static uint32_t pf_rows(uint32_t head_dim) {
-  return 16 * (head_dim == 256 ? kPfRowTiles256 : kPfRowTiles) * kPfWaves;
-}
-
 uint64_t prefill_grid(uint32_t batch, uint32_t kvh, uint32_t group, uint32_t max_q,
                       uint32_t head_dim) {
   const uint64_t rows = pf_rows(head_dim);
   return ((uint64_t)max_q * group + rows - 1) / rows * kvh * batch;
 }
-
-// Key splits for a launch of `base` workgroups (query tiles x kv heads x
-// sequences) over at most max_k keys: enough to give every CU of a 256-CU
-// GPU a workgroup (one workgroup per CU is the kernel's occupancy at
-// head_dim 128), each split keeping at least 8 steps of 32 keys, at most 64.
-static uint32_t pf_splits(uint64_t base, uint32_t max_k) {
-  constexpr uint64_t kTarget = 256;
-  if (base == 0 || base >= kTarget) return 1;
-  uint64_t n = (kTarget + base - 1) / base;
-  n = std::min<uint64_t>(n, std::max<uint32_t>(1u, max_k / 256));
-  return (uint32_t)std::min<uint64_t>(n, 64);
-}
-
-static uint64_t pf_split_bytes(uint64_t base, uint32_t n, uint32_t head_dim,
-                               uint32_t rows = 16 * kPfRowTiles * kPfWaves) {
-  return n > 1 ? base * n * pf_part_bytes(rows, head_dim) : 0;
-}
-
-// At most this much workspace for the partials (fewer splits beyond).
-constexpr uint64_t kPfSplitMaxBytes = 256ull << 20;
-
-static uint32_t pf_splits_within(uint64_t base, uint32_t max_k, uint32_t head_dim,
-                                 uint64_t bytes, uint32_t rows = 16 * kPfRowTiles * kPfWaves) {
-  uint32_t n = pf_splits(base, max_k);
-  while (n > 1 && pf_split_bytes(base, n, head_dim, rows) > std::min(bytes, kPfSplitMaxBytes))
-    --n;
-  return n;
-}
-
-// Ranges of equal work instead of tiles or their n_split equal shares, where
-// what those leave idle is more than the ranges' plan, partials and merge
-// cost (a partial is written and read once; ~ranges + tiles of them against
-// n_split per tile). The host knows the longest sequence only: idle is what
-// the rounds of workgroups leave if all are as long (5% at least). Measured
-// (us, tiles or shares / ranges; bf16, 32 q / 8 kv heads): 3 x 512 queries
-// over 4,096 keys (192 tiles in 384 shares) 150 / 126, 5 x 512 (320 tiles)
-// 242 / 197, 10 chunks of 20-100 over ~1,000 keys 79 / 53; f32, 40 chunks of
-// 16 over ~1,000 keys 378 / 168; and where it says no: 4 x 512 (256 tiles) 135
-// / 154, 1 x 512 (256 shares) 57 / 63, 1 x 1,500 fresh 53 / 73.
-PfRangePlan pf_range_plan(uint64_t items, uint32_t max_q, uint32_t max_k, uint32_t slots,
-                          uint32_t n_split, float step_us, uint64_t part_bytes,
-                          size_t ws_bytes) {
-  constexpr float kMergeUs = 4.f, kPlanUs = 5.f, kMarginUs = 3.f, kBytesPerUs = 5e6f;
-  PfRangePlan p{0, 0};
-  if (items == 0 || items >= 4 * slots) return p;
-  const uint64_t wgs = items * n_split, rounds = (wgs + slots - 1) / slots;
-  const float idle = std::max(1.f - (float)wgs / (float)(rounds * slots), 0.05f);
-  const float steps_now = (float)(max_k - std::min(max_q / 2, max_k)) / 32.f / (float)n_split;
-  const float part_us = 2.f * (float)part_bytes / kBytesPerUs;
-  const float cost = kPlanUs + kMergeUs + part_us * (float)(kPfMaxRanges + items) -
-                     (n_split > 1 ? kMergeUs + part_us * (float)wgs : 0.f);
-  if ((float)rounds * steps_now * step_us * idle < cost + kMarginUs) return p;
-  // The steps there can be, kPfMinSteps to a range; two partials each.
-  const uint64_t steps = items * (max_k / 32 + 2);
-  if (16 * steps > kPfMaxCount) return p;
-  uint64_t n = std::min<uint64_t>(kPfMaxRanges, (steps + kPfMinSteps - 1) / kPfMinSteps);
-  const uint64_t bytes = std::min<uint64_t>(ws_bytes, kPfSplitMaxBytes);
-  if (bytes <= kPfRangeHead) return p;
-  n = std::min<uint64_t>(n, (bytes - kPfRangeHead) / (2 * part_bytes));
-  if (n < 2) return p;
-  p.ranges = (uint32_t)n;
-  p.bytes = kPfRangeHead + n * 2 * part_bytes;
-  return p;
-}
-
-// Launches that may run as ranges: at head_dim 256 the walk over a range's
-// pieces does not fit beside the kernel's registers, and longer lists do not
-// fit the plan; those split every item equally where they split.
-static bool pf_ranges_ok(uint32_t n_seqs, uint32_t head_dim) {
-  return n_seqs <= kPfSortSeqs && head_dim <= 128;
-}
-
-// A full workgroup's 32-key step (head_dim 128; less below).
-constexpr float kPfStepUs = 1.15f;
-// Workgroups of the tiled prefill that the GPU runs at once.
-static uint32_t pf_slots(uint32_t head_dim) { return 256u * (head_dim == 64 ? kPfOcc64 : kPfOcc); }
 
 void launch_prefill_range_merge(const AttnArgs& a, uint32_t ranges, uint32_t rows, uint32_t dtype,
                                 uint32_t head_dim, const void* ws, hipStream_t s) {
@@ -788,33 +691,18 @@ void launch_prefill_merge_f32(const AttnArgs& a, uint32_t qtiles, uint32_t rows_
 size_t prefill_split_bytes(uint32_t batch, uint32_t kvh, uint32_t group, uint32_t head_dim,
                            uint32_t max_q, uint32_t max_k) {
   if (max_q <= 1) return 0;
-  const uint32_t rows = pf_rows(head_dim);
-  const uint64_t base = prefill_grid(batch, kvh, group, max_q, head_dim);
-  const uint32_t n = pf_splits_within(base, max_k, head_dim, ~0ull, rows);
-  const size_t split = (size_t)pf_split_bytes(base, n, head_dim, rows);
-  if (!pf_ranges_ok(batch, head_dim)) return split;
-  return std::max(split, pf_range_plan(base, max_q, max_k, pf_slots(head_dim), n, kPfStepUs,
-                                       pf_part_bytes(rows, head_dim), ~0ull)
-                             .bytes);
+  const PfRoute r = pf_route(batch, kvh, group, max_q, max_k, head_dim, true, ~0ull);
+  return std::max((size_t)pf_split_bytes(r.items, r.n_split, head_dim, r.rows), r.ranges.bytes);
 }
 
 void launch_prefill(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, uint32_t head_dim,
                     bool bf16, void* split_ws, size_t split_ws_bytes, hipStream_t s) {
   AttnArgs a = a_in;
-  const uint32_t rows = pf_rows(head_dim);
-  const uint32_t qtiles = (uint32_t)(((uint64_t)max_q * a.group + rows - 1) / rows);
-  const uint64_t base = (uint64_t)qtiles * a.kvh * a.pf_seqs_n;
-  // As many splits as the workspace given holds (none without one); a
-  // deterministic call does not split, so its output does not depend on
-  // the workspace it is given.
-  const bool split_ok = split_ws && !a.deterministic;
-  const uint32_t n_split =
-      split_ok ? pf_splits_within(base, max_k, head_dim, split_ws_bytes, rows) : 1;
-  const PfRangePlan rp =
-      split_ok && pf_ranges_ok(a.pf_seqs_n, head_dim)
-          ? pf_range_plan(base, max_q, max_k, pf_slots(head_dim), n_split, kPfStepUs,
-                          pf_part_bytes(rows, head_dim), split_ws_bytes)
-          : PfRangePlan{0, 0};
+  const PfRoute route = pf_route(a.pf_seqs_n, a.kvh, a.group, max_q, max_k, head_dim,
+                                 split_ws && !a.deterministic, split_ws_bytes);
+  const uint32_t rows = route.rows, qtiles = route.qtiles, n_split = route.n_split;
+  const uint64_t base = route.items;
+  const PfRangePlan rp = route.ranges;
   a.pf_sort = prefill_sorts(a.pf_seqs_n, qtiles, base * n_split);
   float* part = n_split > 1 ? (float*)split_ws : nullptr;
   const dim3 grid((uint32_t)(base * n_split)), block(kPfThreads);

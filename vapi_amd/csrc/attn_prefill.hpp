@@ -61,54 +61,14 @@ __device__ __forceinline__ uint32_t lds_addr(const uint16_t* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint16_t*)p;
 }
 
-// ---- balanced ranges of a prefill launch ------------------------------------
-//
-// A launch whose query tiles do not fill the GPU's workgroup slots evenly
-// (fewer tiles than slots, or a last round that is nearly empty, or tiles of
-// very different lengths) is cut into ranges of equal work instead, one
-// workgroup each: a range may start and end inside a tile and cover whole
-// tiles between. The tiles' order is kv head, then list order, then each
-// sequence from its last tile to its first; XCD x runs a contiguous eighth of
-// the ranges, so the tiles that run together on an XCD share a kv head's K/V.
-// A tile's work is counted in sixteenths of a 32-key step and falls by a
-// constant from a sequence's last tile to its first (the causal mask; not at
-// all with a window), so sums over tiles have a closed form; a piece's share
-// of that count is then its share of the tile's real steps.
-//
-// The first piece of range r that is not a whole tile goes to partial slot
-// 2 r if it starts the range, else to 2 r + 1. The range that starts a tile
-// without ending it describes the tile (PfSplitTile), and the merge joins its
-// piece with the following ranges' first pieces.
-constexpr uint32_t kPfMinSteps = 8;  // per range, in launches of few steps
-
-struct PfSplitTile {
-  uint32_t valid, seq, qt, kh;
-  uint32_t first_slot, last;  // partial slot of the first piece, the last range
-  uint32_t pad[2];
-};
-
-// The plan, in LDS: one entry per sequence of the list (at most kPfSortSeqs,
-// one per lane while it is made). Every wave makes the same one and reads its
-// own, so no barrier stands between.
-struct PfEntry {
-  uint32_t seq, q0, len_q, len_k;
-  uint32_t nt, c_last, fall;  // tiles, the last tile's count, what each earlier one has less
-  uint32_t pad;
-};
-
-// The step of `steps` at count u of c: 0 at 0, all of them at c, never falling
-// between, the same wherever it is computed.
-__device__ __forceinline__ uint32_t pf_step_at(uint32_t u, uint32_t c, uint32_t steps) {
-  return u >= c ? steps : min(steps, (uint32_t)((float)u * ((float)steps / (float)c)));
-}
-
-__device__ __forceinline__ uint32_t pf_tiles_sum(uint32_t c, uint32_t f, uint32_t n) {
-  return n * c - f * (n * (n - 1) / 2);
-}
+// ---- the walk over a range (prefill_plan.hpp says what ranges are) ------------
 
 // A walk over the plan's tiles: tile m from the last of list entry li's.
 struct PfWalk {
-  PfEntry* plan;   // this wave's
+  // In LDS, one entry per sequence of the list (at most kPfSortSeqs, one per
+  // lane while it is made). Every wave makes the same one and reads its own, so
+  // no barrier stands between.
+  PfEntry* plan;
   PfEntry mine;    // this lane's entry, until the first tile is found
   uint32_t sum;    // and the count of its tiles
   uint64_t some;   // entries with tiles
@@ -127,19 +87,9 @@ struct PfWalk {
         e.q0 = cu_q[e.seq], e.len_q = cu_q[e.seq + 1] - e.q0;
         e.len_k = cu_k[e.seq + 1] - cu_k[e.seq];
         if (e.len_q >= a.pf_min_q && e.len_q > 0)
-          e.nt = min((uint32_t)(((uint64_t)e.len_q * a.group + rows - 1) / rows), qtiles);
+          pf_entry_tiles(e, a.group, qtiles, rows, a.wl, a.wr,
+                         pf_count_cap(qtiles * a.kvh * a.pf_seqs_n));
       }
-    }
-    if (e.nt) {
-      // Steps of the last tile, from its first row's window to its last key.
-      const int32_t offset = (int32_t)(e.len_k - e.len_q);
-      int32_t klo, khi, unused;
-      key_range(offset + (int32_t)((e.nt - 1) * rows / a.group), (int32_t)e.len_k, a.wl, a.wr,
-                klo, unused);
-      key_range(offset + (int32_t)e.len_q - 1, (int32_t)e.len_k, a.wl, a.wr, unused, khi);
-      e.c_last = 16u * (khi >= klo ? (uint32_t)((khi >> 5) - (klo >> 5) + 1) : 1u);
-      if (a.wl < 0 && a.wr >= 0 && e.nt > 1)
-        e.fall = min(rows / (2 * a.group), (e.c_last - 16) / (e.nt - 1));
     }
     mine = e;
     sum = pf_tiles_sum(e.c_last, e.fall, e.nt);
@@ -211,57 +161,34 @@ __device__ __forceinline__ void pf_walk_range(const AttnArgs& a, const uint32_t*
   __shared__ PfEntry entries[64 * W];
   PfWalk w;
   w.init(a, cu_q, cu_k, qtiles, rows, entries);
-  // 32-bit counts: the host takes ranges only where S * ranges fits (lengths
-  // past its max_seqlen_k may wrap it: the walk then ends at the last head).
-  const uint32_t S = w.total * a.kvh;
-  const uint32_t nr = min(ranges, (S + 16 * kPfMinSteps - 1) / (16 * kPfMinSteps));
+  const uint32_t S = w.total * a.kvh, nr = pf_range_count(S, ranges);
   if (bid >= nr || !w.some) {
     if (threadIdx.x == 0) tiles[bid].valid = 0;
     return;
   }
   const uint32_t x = bid % 8, r = x * (nr / 8) + min(x, nr % 8) + bid / 8;
-  uint32_t at = S * r / nr;
-  const uint32_t end = S * (r + 1) / nr;
-  const uint32_t kh0 = at / w.total;
-  uint32_t u0 = w.seek(kh0, at - kh0 * w.total);
-  uint32_t slot = 2 * r, goes_on = 0;
-  while (at < end && w.kh < a.kvh) {
-    const uint32_t c = w.count(), u1 = min(c, u0 + (end - at));
-    const PfItem it = w.item();
-    piece(it, u0, u1, c, u0 == 0 && u1 == c ? ~0u : slot);
-    if (u0 == 0 && u1 < c) {  // starts here, ends in a later range
-      goes_on = 1;
-      if (threadIdx.x == 0) {
-        PfSplitTile t;
-        t.valid = 1, t.seq = it.seq, t.qt = it.qt, t.kh = it.kh, t.first_slot = slot;
-        t.last = min(((at + c) * nr + S - 1) / S, nr) - 1;
-        t.pad[0] = t.pad[1] = 0;
-        tiles[r] = t;
-      }
-    }
-    at += u1 - u0;
-    if (at >= end) break;
-    u0 = 0, slot = 2 * r + 1;
-    w.next();
-    __syncthreads();
-  }
-  if (threadIdx.x == 0 && !goes_on) tiles[r].valid = 0;
+  const bool open = pf_walk_pieces(
+      w, S, nr, r, a.kvh, w.total,
+      [&](uint32_t u0, uint32_t u1, uint32_t c, uint32_t slot) __attribute__((always_inline)) {
+        piece(w.item(), u0, u1, c, slot);
+      },
+      [&]() __attribute__((always_inline)) {
+        w.next();
+        __syncthreads();
+      },
+      [&](uint32_t slot, uint32_t last) __attribute__((always_inline)) {
+        if (threadIdx.x == 0) {
+          const PfItem it = w.item();
+          PfSplitTile t;
+          t.valid = 1, t.seq = it.seq, t.qt = it.qt, t.kh = it.kh, t.first_slot = slot;
+          t.last = last;
+          t.pad[0] = t.pad[1] = 0;
+          tiles[r] = t;
+        }
+      });
+  if (threadIdx.x == 0 && !open) tiles[r].valid = 0;
 }
 
-// The launch's side of it: at most one range per CU; the split tiles lead the
-// workspace, the partials follow.
-constexpr uint32_t kPfMaxRanges = 256;
-constexpr uint64_t kPfMaxCount = 0xFFFFFFFFull / kPfMaxRanges;  // of all tiles
-constexpr size_t kPfRangeHead = kPfMaxRanges * sizeof(PfSplitTile);
-struct PfRangePlan {
-  uint32_t ranges;  // 0: none, the launch runs its tiles as they are
-  size_t bytes;     // of workspace
-};
-// For `items` tiles if every sequence is as long as the longest, of at most
-// max_k keys and max_q queries, which would otherwise run as n_split shares each, `slots` at
-// once, step_us a step; partials of part_bytes each.
-PfRangePlan pf_range_plan(uint64_t items, uint32_t max_q, uint32_t max_k, uint32_t slots,
-                          uint32_t n_split, float step_us, uint64_t part_bytes, size_t ws_bytes);
 void launch_prefill_range_merge(const AttnArgs& a, uint32_t ranges, uint32_t rows, uint32_t dtype,
                                 uint32_t head_dim, const void* ws, hipStream_t s);
 

@@ -59,9 +59,6 @@
 
 namespace vk {
 
-constexpr int kPf32Waves = 8;
-constexpr int kPf32Threads = 64 * kPf32Waves;
-constexpr uint32_t x3_rows(int row_tiles) { return 16u * (uint32_t)row_tiles * kPf32Waves; }
 constexpr int kPfF32Waves = 4;
 
 // Eight (or fewer) values split into three planes of packed bf16.
@@ -644,81 +641,8 @@ __global__ __launch_bounds__(64 * kPfF32Waves, 1) void paged_prefill_f32(
 }
 
 
-constexpr int kPfF32RowTiles = 2;
-constexpr float kX3StepUs = 2.82f;  // a workgroup's 32-key step with one row tile per wave
-
-// The kernel of a launch of n_seqs sequences: rows per item and the items
-// that fill a 256-CU GPU.
-struct F32Plan {
-  bool x3;
-  uint32_t row_tiles;  // per wave
-  uint32_t rows;       // per item: a workgroup's (x3, one per CU) or a wave's
-  uint32_t qtiles;
-  uint64_t items, target;
-};
-static F32Plan f32_plan(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_q) {
-  F32Plan p;
-  const uint64_t all = (uint64_t)max_q * group;
-  // The split kernel from 128 rows per kv head (a full item), and below that
-  // for few kv heads: an item with few rows leaves most of its waves without
-  // MFMAs, so where items fill the GPU four f32 waves per CU go further. Per
-  // call, contexts around 1,000 (x3 against f32 MFMAs): 320 items (40
-  // sequences, 8 kv heads) of 128 rows 500 against 735 us, of 64 rows 492
-  // against 379; 64 items of 12 rows 39 against 54 us, of 64 rows 54 against
-  // 60; 128 items of 64 rows 93 against 90, of 96 rows 114 against 180; 192
-  // items of 13 rows 120 against 102.
-  const uint64_t heads = (uint64_t)kvh * n_seqs;
-  p.x3 = all >= x3_rows(1) || heads <= 64 || (heads <= 128 && all > 64);
-  // Two row tiles per wave halve the LDS reads per MFMA: with enough items
-  // (8 x 512 rows over 4,096 keys, 512 items: 1,148 against 1,457 us with
-  // one row tile); below that the smaller items balance better (4 ragged
-  // chunks of 360-429 over ~2,100 keys, 16 q / 8 kv heads: 192 against 223).
-  auto items = [&](uint64_t rows) { return (all + rows - 1) / rows * kvh * n_seqs; };
-  p.row_tiles = !p.x3 || items(x3_rows(2)) >= 256 ? 2 : 1;
-  p.rows = p.x3 ? x3_rows(p.row_tiles) : 16 * kPfF32RowTiles;
-  p.qtiles = (uint32_t)((all + p.rows - 1) / p.rows);
-  p.items = items(p.rows);
-  p.target = p.x3 ? 256 : 1024;
-  return p;
-}
-
-// The same launch in ranges: one row tile per wave (with two, the walk over a
-// range's pieces does not fit the registers beside the kernel's).
-static F32Plan f32_range_plan(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_q) {
-  F32Plan p = f32_plan(n_seqs, kvh, group, max_q);
-  const uint64_t all = (uint64_t)max_q * group;
-  // (Ranges balance the items that few rows would leave half idle: 40
-  // sequences, 8 kv heads, 64 rows over ~1,000 keys: 378 us with f32 MFMAs.)
-  p.x3 = p.x3 || all > 32;
-  p.row_tiles = 1;
-  p.rows = x3_rows(1);
-  p.qtiles = (uint32_t)((all + p.rows - 1) / p.rows);
-  p.items = (uint64_t)p.qtiles * kvh * n_seqs;
-  return p;
-}
-
 uint64_t prefill_f32_items(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_q) {
   return f32_plan(n_seqs, kvh, group, max_q).items;
-}
-
-// Key splits over at most max_k keys: enough to fill the GPU, each split
-// keeping at least 8 steps of 32 keys, at most 64; fewer when the workspace
-// given holds fewer partials (at most 256 MiB of them).
-static uint32_t pf32_splits(const F32Plan& p, uint32_t max_k, uint32_t head_dim, uint64_t bytes) {
-  if (p.items == 0 || p.items >= p.target) return 1;
-  uint64_t n = std::min<uint64_t>((p.target + p.items - 1) / p.items,
-                                  std::max<uint32_t>(1u, max_k / 256));
-  n = std::min<uint64_t>(n, 64);
-  const uint64_t cap = std::min<uint64_t>(bytes, 256ull << 20);
-  while (n > 1 && p.items * n * pf_part_bytes(p.rows, head_dim) > cap) --n;
-  return (uint32_t)n;
-}
-
-static PfRangePlan f32_ranges(const F32Plan& p, uint32_t n_seqs, uint32_t max_q, uint32_t max_k,
-                              uint32_t head_dim, uint64_t bytes) {
-  if (!p.x3 || n_seqs > kPfSortSeqs) return PfRangePlan{0, 0};
-  return pf_range_plan(p.items, max_q, max_k, 256, pf32_splits(p, max_k, head_dim, bytes),
-                       kX3StepUs, pf_part_bytes(p.rows, head_dim), bytes);
 }
 
 size_t prefill_f32_split_bytes(uint32_t batch, uint32_t kvh, uint32_t group, uint32_t head_dim,
@@ -727,8 +651,8 @@ size_t prefill_f32_split_bytes(uint32_t batch, uint32_t kvh, uint32_t group, uin
   const F32Plan p = f32_plan(batch, kvh, group, max_q);
   const uint32_t n = pf32_splits(p, max_k, head_dim, ~0ull);
   const size_t split = n > 1 ? (size_t)(p.items * n * pf_part_bytes(p.rows, head_dim)) : 0;
-  const F32Plan r = f32_range_plan(batch, kvh, group, max_q);
-  return std::max(split, f32_ranges(r, batch, max_q, max_k, head_dim, ~0ull).bytes);
+  return std::max(split,
+                  f32_route(batch, kvh, group, max_q, max_k, head_dim, true, ~0ull).ranges.bytes);
 }
 
 void launch_prefill_f32(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, uint32_t head_dim,
@@ -736,14 +660,11 @@ void launch_prefill_f32(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, ui
   AttnArgs a = a_in;
   // No split without a workspace, nor for a deterministic call (its output
   // must not depend on the workspace it is given).
-  const bool split_ok = split_ws && !a.deterministic;
-  F32Plan p = f32_range_plan(a.pf_seqs_n, a.kvh, a.group, max_q);
-  const PfRangePlan rp = split_ok ? f32_ranges(p, a.pf_seqs_n, max_q, max_k, head_dim, split_ws_bytes)
-                                  : PfRangePlan{0, 0};
-  if (!rp.ranges) p = f32_plan(a.pf_seqs_n, a.kvh, a.group, max_q);
-  const uint32_t qtiles = p.qtiles;
-  const uint32_t n_split =
-      split_ok && !rp.ranges ? pf32_splits(p, max_k, head_dim, split_ws_bytes) : 1;
+  const F32Route route = f32_route(a.pf_seqs_n, a.kvh, a.group, max_q, max_k, head_dim,
+                                   split_ws && !a.deterministic, split_ws_bytes);
+  const F32Plan& p = route.plan;
+  const PfRangePlan rp = route.ranges;
+  const uint32_t qtiles = p.qtiles, n_split = route.n_split;
   const uint64_t items = p.items * n_split;
   a.pf_sort = prefill_sorts(a.pf_seqs_n, qtiles, items);
   const uint32_t wgs = (uint32_t)((items + kPfF32Waves - 1) / kPfF32Waves);
