@@ -82,3 +82,37 @@ def test_lengths_past_the_hosts_bound_stay_within_the_counts():
         assert r.ranges
         assert check_walk(r, [q] * n, [1 << 24] * n, 32, 8) == 0
         assert check_walk(r, [q] * n, [k] * (n - 1) + [1 << 30], 32, 8) == 0
+
+
+MIB16 = 16 << 20
+
+
+def test_a_small_workspace_does_not_run_a_launch_on_fewer_cus():
+    """16 MiB hold 62 ranges: a launch that fills the GPU with its tiles keeps
+    them, whatever ranges would save with all the workspace asked for."""
+    for n, heads, kvh, q, k in ((5, 32, 8, 512, 4096), (3, 32, 8, 512, 8192),
+                                (6, 28, 4, 1000, 8000)):
+        assert route(False, n, heads, kvh, q, k, 128).ranges == 256
+        assert route(False, n, heads, kvh, q, k, 128, True, MIB16).ranges == 0
+    assert route(True, 5, 16, 8, 512, 4096, 128).ranges == 256
+    assert route(True, 5, 16, 8, 512, 4096, 128, True, MIB16).ranges == 0
+
+
+def test_ranges_of_a_small_workspace_beat_its_tiles_or_shares():
+    """A range's steps are at most those of the rounds of tiles or shares that
+    the same workspace allows, all sequences as long as the longest."""
+    rng = np.random.default_rng(3)
+    taken = 0
+    for _ in range(20000):
+        n, kvh = int(rng.integers(1, 65)), int(rng.choice([1, 2, 4, 8, 32]))
+        heads = kvh * int(rng.choice([1, 4, 7]))
+        q = int(np.exp(rng.uniform(np.log(2), np.log(2000))))
+        k = q + int(np.exp(rng.uniform(0, np.log(30000))))
+        ws = int(np.exp(rng.uniform(np.log(1 << 20), np.log(128 << 20))))
+        r = route(False, n, heads, kvh, q, k, 128, True, ws)
+        if not r.ranges:
+            continue
+        taken += 1
+        rounds = -(-r.items * r.n_split // 256)
+        assert r.items / r.ranges <= rounds / r.n_split, (r, n, q, k, ws)
+    assert taken > 100

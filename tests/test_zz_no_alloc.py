@@ -12,9 +12,10 @@ import numpy as np
 import pytest
 import torch
 
+from prefill_plan import route
 from test_gpu_attention import max_abs, oracle_out, random_case
 from vapi_amd import _lib
-from vapi_amd.attention import ATTN_DETERMINISTIC, PreparedAttention
+from vapi_amd.attention import ATTN_DETERMINISTIC, ATTN_NO_DECODE_ROWS, PreparedAttention
 from vapi_amd.cache import stream_handle
 
 pytestmark = pytest.mark.gpu
@@ -84,6 +85,29 @@ def test_no_alloc_refuses_a_batch_past_its_scratch_and_writes_nothing():
     assert b"scratch" in _lib.lib().vapi_kv_last_error()
     torch.cuda.synchronize()
     assert bool(torch.isnan(out.float()).all())
+
+
+@pytest.mark.parametrize("dtype,heads,lens_q,lens_k", [
+    (torch.bfloat16, 32, [512] * 5, [4096] * 5),            # tiles: ranges would leave CUs idle
+    (torch.float32, 16, [512, 300, 512, 20, 512], [2300, 2000, 900, 2300, 512]),
+    (torch.bfloat16, 32, [130] * 2, [6000, 700]),           # fewer partials than asked for
+], ids=["bf16-n5", "f32-n5", "bf16-n2"])
+def test_no_alloc_prefill_matches_the_oracle(dtype, heads, lens_q, lens_k):
+    """A prefill whose partials want more workspace than the scratch holds."""
+    rng = np.random.default_rng(11)
+    c, q, batch = random_case(rng, dtype, heads, 8, 128, 16, lens_q, lens_k, "HND")
+    asked = _lib.lib().vapi_paged_attention_workspace_size(c.pool, len(lens_q), heads,
+                                                           max(lens_q), max(lens_k))
+    assert asked > _lib.ATTN_SCRATCH_BYTES
+    if len(lens_q) == 5:
+        f32 = dtype == torch.float32
+        shape = (f32, 5, heads, 8, max(lens_q), max(lens_k), 128)
+        assert route(*shape).ranges and not route(*shape, True, _lib.ATTN_SCRATCH_BYTES).ranges
+    prep = PreparedAttention.from_batch(batch, DEV)
+    got = no_alloc(q, c, prep, ATTN_NO_DECODE_ROWS)
+    ref = oracle_out(q, c, 0, batch, q.shape[2] ** -0.5)
+    tol = 1e-5 if dtype == torch.float32 else 2e-2 * float(ref.abs().max())
+    assert max_abs(got, ref) <= tol
 
 
 def first_call_under_capture():

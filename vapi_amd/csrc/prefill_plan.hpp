@@ -209,8 +209,11 @@ inline uint32_t pf_splits_within(uint64_t base, uint32_t max_k, uint32_t head_di
 // Ranges of equal work instead of tiles or their n_split equal shares, where
 // what those leave idle is more than the ranges' plan, partials and merge
 // cost (a partial is written and read once; ~ranges + tiles of them against
-// n_split per tile). The host knows the longest sequence only: idle is what
-// the rounds of workgroups leave if all are as long (5% at least). Measured
+// n_split per tile). A workspace smaller than asked for holds fewer ranges,
+// which leave CUs without one: they are priced as they are, against the shares
+// that the same workspace allows (16 MiB hold 62: 5 x 512 bf16 queries over
+// 4,096 keys 626 us in ranges, 244 in tiles; 3 x 512 over 8,192 751 / 242).
+// Measured
 // (us, tiles or shares / ranges; bf16, 32 q / 8 kv heads): 3 x 512 queries
 // over 4,096 keys (192 tiles in 384 shares) 150 / 126, 5 x 512 (320 tiles)
 // 242 / 197, 10 chunks of 20-100 over ~1,000 keys 79 / 53; f32, 40 chunks of
@@ -222,21 +225,29 @@ inline PfRangePlan pf_range_plan(uint64_t items, uint32_t max_q, uint32_t max_k,
   constexpr float kMergeUs = 4.f, kPlanUs = 5.f, kMarginUs = 3.f, kBytesPerUs = 5e6f;
   PfRangePlan p{0, 0};
   if (items == 0 || items >= 4 * slots) return p;
-  const uint64_t wgs = items * n_split, rounds = (wgs + slots - 1) / slots;
-  const float idle = std::max(1.f - (float)wgs / (float)(rounds * slots), 0.05f);
-  const float steps_now = (float)(max_k - std::min(max_q / 2, max_k)) / 32.f / (float)n_split;
-  const float part_us = 2.f * (float)part_bytes / kBytesPerUs;
-  const float cost = kPlanUs + kMergeUs + part_us * (float)(kPfMaxRanges + items) -
-                     (n_split > 1 ? kMergeUs + part_us * (float)wgs : 0.f);
-  if ((float)rounds * steps_now * step_us * idle < cost + kMarginUs) return p;
   // The steps there can be, kPfMinSteps to a range; two partials each.
   const uint64_t steps = items * (max_k / 32 + 2);
   if (16 * steps > kPfMaxCount) return p;
-  uint64_t n = std::min<uint64_t>(kPfMaxRanges, (steps + kPfMinSteps - 1) / kPfMinSteps);
+  const uint64_t all = std::min<uint64_t>(kPfMaxRanges, (steps + kPfMinSteps - 1) / kPfMinSteps);
   const uint64_t bytes = std::min<uint64_t>(ws_bytes, kPfSplitMaxBytes);
   if (bytes <= kPfRangeHead) return p;
-  n = std::min<uint64_t>(n, (bytes - kPfRangeHead) / (2 * part_bytes));
+  const uint64_t n = std::min<uint64_t>(all, (bytes - kPfRangeHead) / (2 * part_bytes));
   if (n < 2) return p;
+  const uint64_t wgs = items * n_split, rounds = (wgs + slots - 1) / slots;
+  const float steps_now = (float)(max_k - std::min(max_q / 2, max_k)) / 32.f / (float)n_split;
+  const float now_us = (float)rounds * steps_now * step_us;
+  // Time in ranges: all of them divide what the rounds do not leave idle (5%
+  // at least: the host knows the longest sequence only); fewer, for want of
+  // workspace, walk the launch's steps without a share of that (two workgroups
+  // on a CU take as long for a step each as one for two).
+  const float idle = std::max(1.f - (float)wgs / (float)(rounds * slots), 0.05f);
+  const float ranges_us =
+      n == all ? now_us * (1.f - idle)
+               : (float)wgs * steps_now * step_us / (float)n * (float)kPfMaxRanges / (float)slots;
+  const float part_us = 2.f * (float)part_bytes / kBytesPerUs;
+  const float cost = kPlanUs + kMergeUs + part_us * (float)(kPfMaxRanges + items) -
+                     (n_split > 1 ? kMergeUs + part_us * (float)wgs : 0.f);
+  if (now_us - ranges_us < cost + kMarginUs) return p;
   p.ranges = (uint32_t)n;
   p.bytes = kPfRangeHead + n * 2 * part_bytes;
   return p;
