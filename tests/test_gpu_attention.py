@@ -819,6 +819,38 @@ def test_f32_prefill_of_values_without_a_bf16_split(what, det):
     assert float(err.max()) <= 1e-5
 
 
+@pytest.mark.parametrize("rows", ["ranges", "whole", "two_tiles"])
+@pytest.mark.parametrize("what", ["v_columns", "qk_column"])
+def test_f32_prefill_keeps_the_bits_of_small_values_beside_large_ones(what, rows):
+    """Columns whose values bf16 splits would cut short, beside ordinary ones:
+    each V column at the f32 bar of its own scale, and a tiny K column that
+    large queries bring back into the scores."""
+    rng = np.random.default_rng(21)
+    # (Fresh sequences: their first rows average over few keys, or one.)
+    heads, kvh, lens_q, lens_k = {"ranges": (16, 4, [300] * 3, [3000, 300, 300]),
+                                  "whole": (8, 4, [70, 40], [70, 90]),
+                                  "two_tiles": (64, 8, [1100], [1100])}[rows]
+    det = rows != "ranges"  # no split, and two row tiles per wave where there are many
+    r = route(True, len(lens_q), heads, kvh, max(lens_q), max(lens_k), 128, not det)
+    assert bool(r.ranges) == (rows == "ranges")
+    c, q, batch = random_case(rng, torch.float32, heads, kvh, 128, 16, lens_q, lens_k, "HND")
+    unit = torch.ones(128, dtype=torch.float64)
+    if what == "v_columns":
+        for i, e in enumerate((-60, -99, -101, -109, -113, -117, -120, -122)):
+            unit[16 * i + i] = 2.0 ** e
+        c.v[0].mul_(unit.float().to(DEV))
+    else:
+        c.k[0][..., 7] *= 2.0 ** -122
+        q[..., 7] *= 2.0 ** 125
+    want = oracle_out(q, c, 0, batch, 128 ** -0.5)
+    prep = PreparedAttention.from_batch(batch, DEV, cache=c, num_heads=heads,
+                                        deterministic=det)
+    got = torch.full_like(q, float("nan"))
+    paged_attention_prepared(q, c, 0, prep, 128 ** -0.5, out=got)
+    err = ((got.double().cpu() - want.double()) / unit).abs()
+    assert float(err.max()) <= 1e-5, err.amax(dim=(0, 1))[unit < 1]
+
+
 # ---- short decodes: a workgroup (or a few) per sequence and kv head -----------
 
 SMALL_CASES = [

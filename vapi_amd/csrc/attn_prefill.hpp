@@ -57,9 +57,9 @@ __device__ __forceinline__ void ring_barrier() {
   __asm__ volatile("" ::: "memory");
 }
 
-__device__ __forceinline__ uint32_t lds_addr(const uint16_t* p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint16_t*)p;
-}
+// The LDS offset of p: the low half of its flat address. (A cast to the LDS
+// address space would test for null first, inside the loops that use it.)
+__device__ __forceinline__ uint32_t lds_addr(const uint16_t* p) { return (uint32_t)(uintptr_t)p; }
 
 // ---- the walk over a range (prefill_plan.hpp says what ranges are) ------------
 

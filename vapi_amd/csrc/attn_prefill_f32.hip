@@ -19,11 +19,15 @@
 // 1,148 us (105 -> 225 TFLOP/s), the 4 ragged chunks 442 -> 192 us.
 //
 // Values whose h would not be finite (infinities, NaN, |x| above the largest
-// bf16) have no such split, and a tensor of very small values only (all
-// below 2^-100) would lose the low bits of m and l to bf16's exponent range.
-// Every split value is checked as it is made (one packed max per pair); if a
-// workgroup met either, it computes its item again with f32 MFMAs (f32_rows
-// below) and stores that instead.
+// bf16) have no such split: their l is NaN, which reaches every sum that the
+// value is part of, whatever it is multiplied with. And the low bits of m and l
+// of a value below 2^-110 would lie outside bf16's range: the smallest nonzero
+// magnitude is kept as values are split (a shift-add and half a min3 each). If
+// a workgroup ends with a NaN, or met a value that is not zero and below
+// 2^-100, it computes its item again with f32 MFMAs (f32_rows below) and stores
+// that instead. (Probabilities are not checked: one below 2^-110 of its row's
+// largest holds at most 17 good bits already, as the rounding of its exponent
+// is 2^-18 or more.)
 //
 // Rows are the (query token, head) pairs of one kv head, r = j*G + h_local,
 // as in the 16-bit prefill: a workgroup of 8 waves owns 128 RT rows and walks
@@ -65,7 +69,6 @@ constexpr int kPfF32Waves = 4;
 struct Split8 {
   uint4 h, m, l;
 };
-typedef uint16_t ushort2v __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ void split2(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
   h = pack2<bf16_t>(a, b);
@@ -82,34 +85,14 @@ __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
   split2(x[6], x[7], s.h.w, s.m.w, s.l.w);
   return s;
 }
-// Running maximum of |h| over packed pairs (as integers: the order of the
-// magnitudes, infinities and NaN above all finite ones).
-__device__ __forceinline__ void note_magnitude(uint32_t& mag, const uint4& h) {
-  const uint32_t w[4] = {h.x, h.y, h.z, h.w};
+// The smallest 2 |x| - 1 of the bits of the values noted (zeros wrap to the
+// top).
+__device__ __forceinline__ void note_small(uint32_t& small, const float (&x)[8]) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    mag = __builtin_bit_cast(
-        uint32_t, __builtin_elementwise_max(__builtin_bit_cast(ushort2v, mag),
-                                            __builtin_bit_cast(ushort2v, w[i] & 0x7fff7fffu)));
+  for (int i = 0; i < 8; i += 2)
+    small = min(small, min((__float_as_uint(x[i]) << 1) - 1u, (__float_as_uint(x[i + 1]) << 1) - 1u));
 }
-// This wave's notes on one tensor from its lanes' magnitudes: 1 a value that
-// is not finite, 2 one of at least 2^-100, 4 one that is not zero.
-__device__ __forceinline__ uint32_t magnitude_notes(uint32_t mag) {
-  const uint32_t m = max(mag & 0xffffu, mag >> 16);
-  return (__any(m >= 0x7f80u) ? 1u : 0u) | (__any(m >= 0x0d80u) ? 2u : 0u) |
-         (__any(m > 0u) ? 4u : 0u);
-}
-// Whether the workgroup's notes on its three tensors (3 bits each) rule the
-// split out.
-__device__ __forceinline__ bool needs_f32(uint32_t notes) {
-  bool f = false;
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const uint32_t n = (notes >> (3 * i)) & 7u;
-    f = f || (n & 1u) || n == 4u;
-  }
-  return f;
-}
+constexpr uint32_t kSmallest = (0x0d800000u << 1) - 1u;  // 2^-100
 
 // x y over 32 values of k in six MFMAs, the smallest products first.
 __device__ __forceinline__ floatx4 mfma_split(const Split8& x, const Split8& y, floatx4 c) {
@@ -270,7 +253,7 @@ __device__ __forceinline__ void x3_piece(const AttnArgs& a, const uint32_t* __re
   constexpr int kPlaneB = kPlane * 2;
   __shared__ __attribute__((aligned(16))) uint16_t kpl[2][3 * kPlane], vpl[2][3 * kPlane];
   __shared__ uint4 raw[kUnits][2][kPf32Threads];
-  __shared__ uint32_t notes_lds;
+  __shared__ uint32_t outside_lds;
   const uint32_t qt = it.qt, kh = it.kh, q0 = it.q0;
   const uint32_t G = a.group, nrows = it.len_q * G;
   const uint32_t row_base = qt * kPf32Rows;
@@ -333,7 +316,7 @@ __device__ __forceinline__ void x3_piece(const AttnArgs& a, const uint32_t* __re
       __builtin_amdgcn_global_load_lds((const void*)(row + c1), (LdsVoid*)&raw[j][1][64 * wave], 16, 0, 0);
     }
   };
-  uint32_t mag_q = 0, mag_k = 0, mag_v = 0;  // largest |h| of what this thread split
+  uint32_t small = ~0u;  // of what this thread split (note_small)
   // Splits this thread's loaded chunks into the planes of buffer b.
   float4 x0[kUnits], x1[kUnits];
   auto fetch = [&]() __attribute__((always_inline)) {
@@ -351,8 +334,7 @@ __device__ __forceinline__ void x3_piece(const AttnArgs& a, const uint32_t* __re
       const float x[8] = {x0[j].x, x0[j].y, x0[j].z, x0[j].w, x1[j].x, x1[j].y, x1[j].z, x1[j].w};
       const Split8 s = split8(x);
       const uint32_t wr = wr0 + kRowsPerJ * j;
-      if (wr >= 32) note_magnitude(mag_v, s.h);
-      else note_magnitude(mag_k, s.h);
+      note_small(small, x);
       uint16_t* dst = (wr >= 32 ? vpl[b] : kpl[b]) + pf_chunk<D>((row0_ + kRowsPerJ * j) & 31, pos);
       *(uint4*)dst = s.h;
       *(uint4*)(dst + kPlane) = s.m;
@@ -386,7 +368,7 @@ __device__ __forceinline__ void x3_piece(const AttnArgs& a, const uint32_t* __re
                           __uint_as_float(v.x ^ sg), __uint_as_float(v.y ^ sg),
                           __uint_as_float(v.z ^ sg), __uint_as_float(v.w ^ sg)};
       qf[t][c] = split8(x);
-      note_magnitude(mag_q, qf[t][c].h);
+      note_small(small, x);
     }
   }
   float m_run[RT], l_run[RT];
@@ -509,16 +491,24 @@ __device__ __forceinline__ void x3_piece(const AttnArgs& a, const uint32_t* __re
   }
   wait_vmcnt<0>();  // no load may land in LDS after the workgroup ends
 
-  // Values without a split anywhere in the workgroup's share: f32 MFMAs.
-  if (tid == 0) notes_lds = 0;
+  // Values without a split anywhere in the workgroup's share: f32 MFMAs. (NaN
+  // is looked for in the bits: the build's float compares assume there is none.)
+  if (tid == 0) outside_lds = 0;
   __syncthreads();
   {
-    const uint32_t notes =
-        magnitude_notes(mag_q) | magnitude_notes(mag_k) << 3 | magnitude_notes(mag_v) << 6;
-    if (lane == 0) atomicOr(&notes_lds, notes);
+    uint32_t top = 0;
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      top = max(top, __float_as_uint(l_run[t]) << 1);
+#pragma unroll
+      for (int k = 0; k < DL; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) top = max(top, __float_as_uint(o[t][k][i]) << 1);
+    }
+    if (__any(small < kSmallest || top > (0x7f800000u << 1)) && lane == 0) outside_lds = 1;
   }
   __syncthreads();
-  if (needs_f32(__builtin_amdgcn_readfirstlane(notes_lds))) {
+  if (__builtin_amdgcn_readfirstlane(outside_lds)) {
 #pragma unroll 1
     for (uint32_t t = 0; t < (uint32_t)RT; ++t)
       f32_rows<D, 1, kPad, D / 16, false>(a, tab, kh, q0, nrows, row0 + 16 * t, offset, len_k, klo,
