@@ -19,7 +19,7 @@ from test_gpu_attention import max_abs, oracle_out, random_case
 from vapi_amd import _lib, workload
 from vapi_amd.attention import (ForwardBatch, PreparedAttention,
                                 paged_attention_append_prepared, paged_attention_prepared)
-from vapi_amd.cache import PagedKvCache, write_rows_indexed
+from vapi_amd.cache import PagedKvCache, stream_handle, write_rows_indexed
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -157,7 +157,7 @@ def test_fused_step_over_more_rows_than_one_launch_plans_for():
 
 @pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.float32, 128)])
 def test_a_decode_grows_a_workspace_that_is_too_small(dtype, d):
-    """The library refuses the small one before it writes anything."""
+    """Whether the append is fused with the attention (bf16) or not (f32)."""
     rng = np.random.default_rng(5)
     lens_k = [900, 40, 3000]
     c, q, batch = random_case(rng, dtype, 8, 2, d, 16, [1] * 3, lens_k, "HND")
@@ -172,3 +172,30 @@ def test_a_decode_grows_a_workspace_that_is_too_small(dtype, d):
         small.workspace = torch.zeros(256, dtype=torch.uint8, device=DEV)
         assert torch.equal(fn(small), want)
         assert small.workspace.numel() == size
+
+
+@pytest.mark.parametrize("dtype,d,lens_q", [(torch.bfloat16, 128, [1, 1]), (torch.bfloat16, 96, [1, 1]),
+                                            (torch.float32, 128, [1, 1]),
+                                            (torch.float32, 64, [1, 30])])
+def test_an_append_refused_for_its_workspace_writes_nothing(dtype, d, lens_q):
+    """Through the C entry, fused or not: the pool is as it was."""
+    rng = np.random.default_rng(8)
+    c, q, batch = random_case(rng, dtype, 8, 2, d, 16, lens_q, [900, 3000], "HND")
+    n = sum(lens_q)
+    k_new, v_new = new_rows(n, 2, d, dtype, 9)
+    s = dev_slots(step_slots(batch, 16))
+    prep = PreparedAttention.from_batch(batch, DEV)
+    before = [c.k[0].clone(), c.v[0].clone()]
+    out = torch.full_like(q, float("nan"))
+    ws = torch.zeros(256, dtype=torch.uint8, device=DEV)
+    lib = _lib.lib()
+    for ptr, size in ((ws.data_ptr(), 256), (None, 0), (None, 1 << 30)):
+        rc = lib.vapi_paged_attention_append_ex(
+            c.pool, 0, k_new.data_ptr(), v_new.data_ptr(), s.data_ptr(), n, q.data_ptr(),
+            out.data_ptr(), prep.seqlens_q.data_ptr(), prep.seqlens_k.data_ptr(),
+            prep.block_table.data_ptr(), 2, prep.block_table.shape[1], max(lens_q), 3000, 8,
+            d ** -0.5, -1, 0, 0, ptr, size, stream_handle())
+        assert rc == _lib.ESPACE
+    torch.cuda.synchronize()
+    assert torch.equal(c.k[0], before[0]) and torch.equal(c.v[0], before[1])
+    assert bool(torch.isnan(out.float()).all())

@@ -195,6 +195,16 @@ static size_t required_workspace(const vapi_kv_pool* pool, uint32_t batch, uint3
   return skip_decode ? 0 : decode_ws_for(pool, batch, num_heads);
 }
 
+// A batch the caller says has no decode rows (and which is not a fused decode
+// step) runs one kernel: the prefill kernel then takes every row, len_q == 1
+// included, so the result does not depend on the hint. It needs no workspace.
+static bool skips_decode(const vapi_kv_pool* pool, uint32_t batch, uint32_t num_heads,
+                         uint32_t max_seqlen_q, uint32_t max_seqlen_k, bool fused, uint32_t flags) {
+  return (flags & VAPI_ATTN_NO_DECODE_ROWS) && !fused && max_seqlen_q > 1 &&
+         (mfma16_ok(pool, num_heads) ||
+          f32_mfma_ok(pool, num_heads, max_seqlen_q, max_seqlen_k, batch));
+}
+
 // The optional part of the workspace: the prefill key split's partials for
 // n_prefill sequences with prefill rows (a batch of `batch`).
 static size_t split_bytes(const vapi_kv_pool* pool, uint32_t batch, uint32_t num_heads,
@@ -317,6 +327,16 @@ int vapi_paged_attention_append_ex(const vapi_kv_pool* pool, uint32_t layer, con
                      num_heads % pool->num_kv_heads == 0 && mfma_ok(pool, num_heads) &&
                      num_heads / pool->num_kv_heads <= 16;
   if (!fused) {
+    // A workspace too small is refused before the append is launched (a
+    // refused call writes nothing).
+    if (batch > 0 && max_seqlen_q > 0 && num_heads > 0 && num_heads % pool->num_kv_heads == 0) {
+      const size_t need = required_workspace(
+          pool, batch, num_heads, max_seqlen_q, max_seqlen_k,
+          skips_decode(pool, batch, num_heads, max_seqlen_q, max_seqlen_k, false, flags));
+      if (workspace_bytes < need || (need && !workspace))
+        VK_FAIL(VAPI_KV_ESPACE, "vapi_paged_attention_append: workspace %zu bytes < %zu",
+                workspace_bytes, need);
+    }
     if (int rc = vapi_kv_append(pool, layer, k_src, v_src, slot_mapping, n_tokens, stream))
       return rc;
     return vapi_paged_attention_ex(pool, layer, q, out, cu_seqlens_q, cu_seqlens_k, block_table,
@@ -394,13 +414,8 @@ static int paged_attention_impl(const vapi_kv_pool* pool, uint32_t layer, const 
        !f32_mfma_ok(pool, num_heads, max_seqlen_q, max_seqlen_k, batch)))
     VK_FAIL(VAPI_KV_EUNSUP, "vapi_paged_attention: batch %u / heads %u too large",
             batch, num_heads);
-  // A batch the caller says has no decode rows (and which is not a fused
-  // decode step) runs one kernel: the prefill kernel then takes every row,
-  // len_q == 1 included, so the result does not depend on the hint. It needs
-  // no workspace.
-  const bool skip_decode = (flags & VAPI_ATTN_NO_DECODE_ROWS) && !fuse && max_seqlen_q > 1 &&
-                           (mfma16_ok(pool, num_heads) ||
-                            f32_mfma_ok(pool, num_heads, max_seqlen_q, max_seqlen_k, batch));
+  const bool skip_decode = skips_decode(pool, batch, num_heads, max_seqlen_q, max_seqlen_k,
+                                        fuse != nullptr, flags);
   // The sequences the prefill grid covers: those the host named (a mixed
   // step's few prefill chunks among many decode rows), else all of them. A
   // prefill-only call covers every row and ignores the list.
