@@ -241,9 +241,15 @@ def test_copy_blocks_rejects_overlapping_pairs():
 
 def test_back_to_back_copies_on_two_streams_see_their_streams_earlier_work():
     """copy_blocks does not wait for the GPU: each call's pairs still reach
-    the launch they belong to, on the current stream and on a given one."""
+    the launch they belong to, on the current stream and on a given one, by
+    torch's object or any other that holds its handle."""
     side = torch.cuda.Stream()
-    for stream in (None, side):
+
+    class Handle:
+        def __init__(self, cuda_stream):
+            self.cuda_stream = cuda_stream
+
+    for stream in (None, side, Handle(side.cuda_stream), Handle(0)):
         c = PagedKvCache(2, 400, 16, 4, 128, torch.bfloat16)
         for l in range(2):
             c.k[l][0] = l + 1.0

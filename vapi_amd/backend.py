@@ -37,6 +37,17 @@ def _dev_u32_async(values: np.ndarray, device) -> torch.Tensor:
     return host.to(device, non_blocking=True)
 
 
+def _torch_stream(stream, device):
+    """`stream` as torch takes it: None (the current one), torch's own, or any
+    other object with a `cuda_stream` handle."""
+    if stream is None or isinstance(stream, torch.cuda.Stream):
+        return stream
+    handle = stream.cuda_stream
+    if handle == 0:  # an ExternalStream of 0 would be a new stream
+        return torch.cuda.default_stream(device)
+    return torch.cuda.ExternalStream(handle, device=device)
+
+
 def _flat_pairs(pairs) -> list | np.ndarray:
     """(source, destination) pairs one after the other, as int64; as a list
     of ints if one of them does not fit."""
@@ -125,7 +136,7 @@ class KvBlockBackend:
         dsts = flat[1::2].tolist()
         if len(set(dsts)) != n or not set(flat[::2].tolist()).isdisjoint(dsts):
             raise ValueError("copy_blocks: destinations must be distinct and not sources")
-        with torch.cuda.stream(stream):  # (None: the current stream)
+        with torch.cuda.stream(_torch_stream(stream, self.cache.device)):
             d_pairs = _dev_u32_async(flat, self.cache.device)
         check(lib().vapi_kv_copy_blocks(self.cache.pool, d_pairs.data_ptr(), n,
                                         stream_handle(stream)))
