@@ -60,6 +60,24 @@ NO_SCRATCH = {"attn_prefill.hip": ("paged_prefill_tiled", "paged_mixed_stream"),
               "attn_decode_small.hip": ("paged_decode_small",),
               "attn_prefill_f32.hip": ("paged_prefill_f32",)}
 
+# Half of a CU's 160 KiB of LDS less the dynamic part (4 bytes for each of the
+# 4,000 sequences that the launch takes, and one more): a workgroup of the mixed
+# step's decode and one of its prefill share a CU.
+MAX_STATIC_LDS = {"attn_prefill.hip": ("paged_mixed_stream", 160 * 1024 // 2 - 4 * 4001)}
+
+
+def _check_static_lds(src: Path, remarks: str) -> None:
+    kernel, most = MAX_STATIC_LDS.get(src.name, ("", 0))
+    current = ""
+    for line in remarks.splitlines():
+        if "Function Name:" in line:
+            current = line.split("Function Name:")[1].split()[0]
+        elif "LDS Size" in line and kernel and kernel in current:
+            size = int(line.split("LDS Size [bytes/block]:")[1].split()[0])
+            if size > most:
+                raise RuntimeError(f"{current} uses {size} bytes of static LDS; two workgroups "
+                                   f"share a CU up to {most}")
+
 
 def _check_no_scratch(src: Path, remarks: str) -> None:
     kernels = NO_SCRATCH.get(src.name)
@@ -87,6 +105,7 @@ def _compile(src: Path, obj: Path) -> None:
         sys.stderr.write(res.stdout + res.stderr)
         raise RuntimeError(f"hipcc failed on {src.name}")
     _check_no_scratch(src, res.stderr)
+    _check_static_lds(src, res.stderr)
 
 
 def _link(objs, out: Path) -> None:

@@ -504,7 +504,8 @@ static int paged_attention_impl(const vapi_kv_pool* pool, uint32_t layer, const 
     const bool room = workspace && workspace_bytes > off;
     // Decode rows and prefill rows in one step: both kernels in one launch.
     // (At most 4,000 sequences: the launch's dynamic LDS, 4 bytes per
-    // sequence, then still lets a decode and a prefill workgroup share a CU.
+    // sequence, then still lets a decode and a prefill workgroup share a CU;
+    // vapi_amd/build.py holds the kernel's static LDS to that.
     // At head_dim 256 neither kernel fits half a CU's registers; a padded
     // head_dim below 128 runs the padded kernels.)
     const bool mixed = !skip_decode && !fuse && parts == 1 && D <= 128 &&

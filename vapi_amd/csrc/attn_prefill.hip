@@ -374,7 +374,8 @@ __device__ __forceinline__ void prefill_piece(const AttnArgs& a, const uint32_t*
   }
 }
 
-// Workgroup `bid` of a prefill launch. With n_split > 1 the steps of each
+// Workgroup `bid` of a prefill launch (`order`: 64 W words of LDS for
+// prefill_item). With n_split > 1 the steps of each
 // item are cut into n_split equal runs, one workgroup each, and
 // paged_prefill_merge combines their partials. Item order: kv head fastest,
 // then key split, then query tile (the items of one tile stay together).
@@ -382,10 +383,9 @@ template <typename T, int D, int RT, int W, bool kSplit, bool kPad = false, int 
 __device__ __forceinline__ void prefill_body(
     const AttnArgs& a, const uint32_t* __restrict__ cu_q, const uint32_t* __restrict__ cu_k,
     const uint32_t* __restrict__ table, uint32_t qtiles, uint32_t n_split_arg,
-    float* __restrict__ part, uint32_t bid) {
+    float* __restrict__ part, uint32_t bid, uint32_t* order) {
   constexpr uint32_t kRows = 16 * RT * W;
   const uint32_t n_split = kSplit ? n_split_arg : 1u;
-  __shared__ uint32_t order[64 * W];
   const uint32_t hr = bid / a.kvh, split = hr % n_split;
   PfItem it;
   if (!prefill_item<W>(a, cu_q, cu_k, (hr / n_split) * a.kvh + bid % a.kvh, qtiles, kRows, order,
@@ -403,8 +403,9 @@ __global__ __launch_bounds__(kPfThreads, OCC) void paged_prefill_tiled(
     AttnArgs a, const uint32_t* __restrict__ cu_q, const uint32_t* __restrict__ cu_k,
     const uint32_t* __restrict__ table, uint32_t qtiles, uint32_t n_split_arg,
     float* __restrict__ part) {
+  __shared__ uint32_t order[64 * kPfWaves];
   prefill_body<T, D, RT, kPfWaves, kSplit, kPad, DL>(a, cu_q, cu_k, table, qtiles, n_split_arg, part,
-                                           blockIdx.x);
+                                           blockIdx.x, order);
 }
 
 // The same over ranges of equal work (see attn_prefill.hpp).
@@ -587,7 +588,7 @@ __global__ __launch_bounds__(256, 2) void paged_mixed_stream(AttnArgs a, uint32_
     decode_stream_body<T, D, false, kPad>(a, a.cu_q, a.cu_k, a.table, P, blockIdx.x, nwg);
   else {
     prefill_body<T, D, kMixRowTiles, kMixPfWaves, kSplit, kPad>(a, a.cu_q, a.cu_k, a.table, qtiles,
-                                                          n_split, part, blockIdx.x - nwg);
+                                                          n_split, part, blockIdx.x - nwg, P);
   }
 }
 
@@ -632,7 +633,8 @@ void launch_mixed(const AttnArgs& a_in, void* workspace, uint32_t max_q, uint32_
   c.pf_sort = prefill_sorts(c.pf_seqs_n, qtiles, base * n_split);
   float* part = n_split > 1 ? (float*)split_ws : nullptr;
   const dim3 grid((uint32_t)(nwg + base * n_split)), block(256);
-  const size_t lds = (c.batch + 1) * sizeof(uint32_t);
+  // The decode's plan, or the prefill's order: one or the other per workgroup.
+  const size_t lds = std::max(c.batch + 1, 64u * kMixPfWaves) * sizeof(uint32_t);
   bool wide = false;
   const uint32_t merge_wgs = decode_merge_wgs(c.batch, c.kvh, &wide);
 #define VK_MIX(T, DD, PAD)                                                                    \
