@@ -10,13 +10,13 @@ using namespace vk;
 extern "C" {
 
 // out: items, query tiles, n_split, ranges, workspace bytes of the ranges,
-// whether the items are sorted.
+// the items' order (PfOrder).
 void plan_route16(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_q, uint32_t max_k,
                   uint32_t head_dim, int split_ok, uint64_t ws_bytes, uint64_t* out) {
   const PfRoute r = pf_route(n_seqs, kvh, group, max_q, max_k, head_dim, split_ok, ws_bytes);
   out[0] = r.items, out[1] = r.qtiles, out[2] = r.n_split, out[3] = r.ranges.ranges;
   out[4] = r.ranges.bytes;
-  out[5] = prefill_sorts(n_seqs, r.qtiles, r.items * r.n_split);
+  out[5] = prefill_order(n_seqs, kvh, r.qtiles, r.items, r.n_split);
 }
 
 void plan_route_f32(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_q, uint32_t max_k,
@@ -24,7 +24,7 @@ void plan_route_f32(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_
   const F32Route r = f32_route(n_seqs, kvh, group, max_q, max_k, head_dim, split_ok, ws_bytes);
   out[0] = r.plan.items, out[1] = r.plan.qtiles, out[2] = r.n_split, out[3] = r.ranges.ranges;
   out[4] = r.ranges.bytes;
-  out[5] = prefill_sorts(n_seqs, r.plan.qtiles, r.plan.items * r.n_split);
+  out[5] = prefill_order(n_seqs, kvh, r.plan.qtiles, r.plan.items, r.n_split);
 }
 
 }  // extern "C"
@@ -135,6 +135,54 @@ extern "C" int plan_check_walk(uint32_t n_seqs, const uint32_t* lens_q, const ui
       if (p.slot >= used.size() || used[p.slot]++) return 14;
     }
     if (at != c || step != steps) return 15;
+  }
+  return 0;
+}
+
+// The order of a sorted launch's tiles as prefill_item finds it, rank by rank:
+// 0 if every tile comes once. `order` takes (sequence, tile) pairs.
+extern "C" int plan_order(uint32_t n, const uint32_t* key, const uint32_t* nt, uint32_t step,
+                          uint32_t* order) {
+  uint32_t longest = 0, tiles = 0;
+  bool classes = false;
+  for (uint32_t s = 0; s < n; ++s)
+    if (nt[s]) longest = pf_max(longest, key[s]), tiles += nt[s];
+  for (uint32_t s = 0; s < n; ++s) classes = classes || pf_short_tile(longest, key[s], nt[s], step);
+  std::vector<std::vector<char>> seen(n);
+  for (uint32_t s = 0; s < n; ++s) seen[s].assign(nt[s], 0);
+  auto to = [&](uint32_t c, uint32_t s) {
+    return pf_tiles_to_class(c, longest, key[s], nt[s], 1.f / (float)step);
+  };
+  for (uint32_t rank = 0; rank < tiles; ++rank) {
+    std::vector<uint32_t> first(n, 0), here(nt, nt + n);
+    uint32_t before = 0;
+    if (classes) {
+      uint32_t c = 0;
+      for (;; ++c) {
+        uint32_t sum = 0;
+        for (uint32_t s = 0; s < n; ++s) sum += to(c, s);
+        if (rank < sum || c + 1 >= kPfClasses) break;
+        before = sum;
+        for (uint32_t s = 0; s < n; ++s) first[s] = to(c, s);
+      }
+      for (uint32_t s = 0; s < n; ++s) {
+        if (to(c, s) < first[s] || to(c, s) > nt[s]) return 1;
+        here[s] = to(c, s) - first[s];
+      }
+    }
+    const uint32_t at = rank - before;
+    int hits = 0;
+    for (uint32_t s = 0; s < n; ++s) {
+      uint32_t start = 0;
+      for (uint32_t o = 0; o < n; ++o)
+        start += key[o] > key[s] || (key[o] == key[s] && o < s) ? here[o] : 0u;
+      if (at < start || at - start >= here[s]) continue;
+      ++hits;
+      const uint32_t m = first[s] + (at - start);
+      if (seen[s][m]++) return 2;
+      order[2 * rank] = s, order[2 * rank + 1] = nt[s] - 1 - m;
+    }
+    if (hits != 1) return 3;
   }
   return 0;
 }

@@ -7,6 +7,7 @@ from functools import lru_cache
 from pathlib import Path
 
 ANY_BYTES = (1 << 64) - 1
+LIST_ORDER, SEQUENCES, PARTS, BY_CLASS = range(4)  # PfOrder
 
 
 @lru_cache(maxsize=None)
@@ -27,7 +28,7 @@ class Route:
     n_split: int
     ranges: int
     range_bytes: int
-    sorts: bool
+    order: int
     rows: int
 
 
@@ -40,7 +41,7 @@ def route(f32, n_seqs, heads, kvh, max_q, max_k, head_dim, split_ok=True, ws_byt
     fn(u32(n_seqs), u32(kvh), u32(heads // kvh), u32(max_q), u32(max_k), u32(head_dim),
        int(split_ok), ctypes.c_uint64(ws_bytes), out)
     rows = 128 if f32 or head_dim == 256 else 256
-    return Route(out[0], out[1], out[2], out[3], out[4], bool(out[5]), rows)
+    return Route(out[0], out[1], out[2], out[3], out[4], out[5], rows)
 
 
 def check_walk(r, lens_q, lens_k, heads, kvh, wl=-1, wr=0):
@@ -52,3 +53,13 @@ def check_walk(r, lens_q, lens_k, heads, kvh, wl=-1, wr=0):
                                   ctypes.c_uint32(heads // kvh), ctypes.c_uint32(r.rows),
                                   ctypes.c_uint32(r.qtiles), ctypes.c_int32(wl),
                                   ctypes.c_int32(wr), ctypes.c_uint32(r.ranges))
+
+
+def tile_order(lens_k, tiles, step):
+    """The (sequence, tile) pairs of a launch by classes, in its order."""
+    n, total = len(lens_k), sum(tiles)
+    out = (ctypes.c_uint32 * (2 * total))()
+    bad = _lib().plan_order(ctypes.c_uint32(n), (ctypes.c_uint32 * n)(*lens_k),
+                            (ctypes.c_uint32 * n)(*tiles), ctypes.c_uint32(step), out)
+    assert bad == 0, bad
+    return [(out[2 * i], out[2 * i + 1]) for i in range(total)]

@@ -16,7 +16,7 @@ import pytest
 import torch
 
 import oracle
-from prefill_plan import route
+from prefill_plan import BY_CLASS, LIST_ORDER, PARTS, SEQUENCES, route
 from vapi_amd import _lib, workload
 from vapi_amd.attention import (ForwardBatch, PreparedAttention, paged_attention,
                                 paged_attention_prepared, paged_attention_windowed)
@@ -712,41 +712,57 @@ def test_small_prefill_batches_split_their_keys_and_match_the_oracle(case):
 # ---- the order of a prefill launch's work items -------------------------------
 
 ORDER_CASES = [
-    # dtype, heads, kvh, d, n_seqs: tiles of 256 rows (128 at head_dim 256)
-    (torch.bfloat16, 4, 1, 64, 2),     # two sequences
-    (torch.float16, 21, 3, 128, 9),    # kv heads that do not divide the XCDs
-    (torch.bfloat16, 32, 8, 128, 64),  # one sequence per lane
-    (torch.bfloat16, 16, 2, 64, 65),   # past the sort: list order
-    (torch.bfloat16, 8, 2, 256, 5),
-    # More items than CUs, so sorted (few items keep list order):
-    (torch.bfloat16, 64, 64, 64, 2),
-    (torch.float16, 21, 3, 128, 40),
-    (torch.bfloat16, 32, 8, 256, 12),
+    # dtype, heads, kvh, d, n_seqs (tiles of 256 rows, 128 at head_dim 256), keys
+    # before the chunks, the order of the prefill-only launch
+    (torch.bfloat16, 4, 1, 64, 2, 0, LIST_ORDER),     # two sequences
+    (torch.float16, 21, 3, 128, 9, 0, LIST_ORDER),    # kv heads that do not divide the XCDs
+    (torch.bfloat16, 32, 8, 128, 64, 0, SEQUENCES),   # one sequence per lane
+    (torch.bfloat16, 16, 2, 64, 65, 0, LIST_ORDER),   # past the sort: list order
+    (torch.bfloat16, 8, 2, 256, 5, 0, LIST_ORDER),
+    # Few items keep list order; more than CUs are sorted:
+    (torch.bfloat16, 64, 64, 64, 2, 0, SEQUENCES),
+    (torch.float16, 21, 3, 128, 40, 0, LIST_ORDER),   # 240 items
+    (torch.float16, 21, 3, 128, 43, 0, SEQUENCES),    # 258
+    (torch.bfloat16, 32, 8, 256, 12, 0, SEQUENCES),
+    # One or two kv heads: by classes of work, or contiguous parts.
+    (torch.bfloat16, 32, 2, 128, 64, 0, BY_CLASS),
+    (torch.float16, 32, 2, 64, 64, 900, BY_CLASS),    # contexts about equal: parts
+    (torch.bfloat16, 48, 2, 256, 50, 600, BY_CLASS),
+    (torch.float32, 16, 2, 128, 64, 0, BY_CLASS),
+    (torch.bfloat16, 64, 2, 128, 3, 0, PARTS),        # chunks of a thousand rows and more
 ]
 
 
-@pytest.mark.parametrize("case", ORDER_CASES, ids=lambda c: f"{str(c[0])[6:]}-kvh{c[2]}-d{c[3]}-n{c[4]}")
+@pytest.mark.parametrize("case", ORDER_CASES,
+                         ids=lambda c: f"{str(c[0])[6:]}-kvh{c[2]}-d{c[3]}-n{c[4]}-k{c[5]}")
 def test_every_tile_of_a_ragged_prefill_batch_is_computed_once(case):
     """Prefill batches of very different lengths (one tile beside several,
     equal contexts, decode rows between them when a list names the prefill
     ones) match the oracle whatever order the launch walks the tiles in."""
-    dtype, heads, kvh, d, n = case
+    dtype, heads, kvh, d, n, before, order = case
     rng = np.random.default_rng(zlib.crc32(str(case).encode()))
+    f32 = dtype == torch.float32
     rows = 128 if d == 256 else 256
     tile = rows * kvh // heads  # query tokens per tile
     lens_q = [int(x) for x in rng.integers(2, tile + 3, n)]
     lens_q[0], lens_q[-1] = 2 * tile + 1, tile
-    lens_k = [l + int(x) for l, x in zip(lens_q, rng.integers(0, 40, n))]
+    if order == PARTS:
+        lens_q = [180 * tile + int(x) for x in rng.integers(0, 2 * tile, n)]
+    lens_k = [before + l + int(x) for l, x in zip(lens_q, rng.integers(0, 40, n))]
     lens_k[-1] = max(lens_k[0], lens_q[-1])  # equal contexts: a tie in the order
     for decode_rows in (False, True):
         if decode_rows:
             lens_q[n // 2] = 1
         c, q, batch = random_case(rng, dtype, heads, kvh, d, 16, lens_q, lens_k, "HND")
-        prep = PreparedAttention.from_batch(batch, DEV, cache=c, num_heads=heads)
+        prep = PreparedAttention.from_batch(batch, DEV, cache=c, num_heads=heads,
+                                            deterministic=f32)  # (no ranges)
+        if not decode_rows:
+            assert route(f32, n, heads, kvh, max(lens_q), max(lens_k), d, not f32).order == order
         want = oracle_out(q, c, 0, batch, d ** -0.5)
         got = torch.full_like(q, float("nan"))
         paged_attention_prepared(q, c, 0, prep, d ** -0.5, out=got)
-        tol = (2e-2 if dtype == torch.bfloat16 else 1e-2) * float(want.abs().max())
+        tol = (1e-5 if f32 else
+               (2e-2 if dtype == torch.bfloat16 else 1e-2) * float(want.abs().max()))
         assert max_abs(got, want) <= tol
 
 

@@ -1,10 +1,12 @@
 """The plan of prefill launches that run as ranges of equal work, on the CPU:
 every range walked with the kernel's own arithmetic, each tile's counts
 covered once, each split tile's description naming its pieces."""
+import heapq
+
 import numpy as np
 import pytest
 
-from prefill_plan import check_walk, route
+from prefill_plan import BY_CLASS, check_walk, route, tile_order
 
 
 def equal(f32, n, heads, kvh, q, k, d=128):
@@ -116,3 +118,55 @@ def test_ranges_of_a_small_workspace_beat_its_tiles_or_shares():
         rounds = -(-r.items * r.n_split // 256)
         assert r.items / r.ranges <= rounds / r.n_split, (r, n, q, k, ws)
     assert taken > 100
+
+
+def test_a_launch_by_classes_takes_every_tile_once_from_the_longest_down():
+    """Over ragged batches: no tile comes before one that has two classes (of
+    16) more work, and tiles of nearly equal work keep their sequences together."""
+    rng = np.random.default_rng(5)
+    for i in range(300):
+        n, step = int(rng.integers(2, 65)), int(rng.choice([1, 3, 16, 36, 64, 256]))
+        top = int(np.exp(rng.uniform(np.log(step), np.log(30000))))
+        lens_q = [int(x) for x in rng.integers(0, min(top, 40 * step) + 1, n)]
+        lens_k = [q + int(x) for q, x in zip(lens_q, rng.integers(0, top + 1, n))]
+        if i % 3 == 0:
+            lens_k = lens_q
+        tiles = [-(-q // step) for q in lens_q]
+        if sum(tiles) > 700:
+            continue
+        order = tile_order(lens_k, tiles, step)
+        work = [lens_k[s] - (tiles[s] - 1 - t) * step for s, t in order]
+        longest = max([k for k, t in zip(lens_k, tiles) if t] + [1])
+        if min(work + [longest]) < longest // 2:
+            after = -10 ** 9
+            for w in reversed(work):  # (thresholds are multiples of longest // 16)
+                assert w >= after - 2 * (longest // 16) - 16
+                after = max(after, w)
+        else:
+            assert order == sorted(order, key=lambda x: (-lens_k[x[0]], x[0], -x[1]))
+
+
+def rounds(order, lens_k, tiles, step, kvh, cus=32):
+    """When the last CU of an XCD ends, in keys, its tiles dealt in order."""
+    end = 0
+    items = [(s, t) for s, t in order for _ in range(kvh)]
+    for x in range(8):
+        free = [0] * cus
+        for s, t in items[x::8]:
+            heapq.heapreplace(free, free[0] + lens_k[s] - (tiles[s] - 1 - t) * step)
+        end = max(end, max(free))
+    return end
+
+
+@pytest.mark.parametrize("heads,kvh,n", [(16, 2, 4), (16, 2, 3), (8, 1, 8), (32, 1, 3)])
+def test_equal_fresh_prompts_end_within_a_quarter_of_an_even_division(heads, kvh, n):
+    """With one or two kv heads, where whole sequences one after the other
+    ended up to half past it."""
+    assert route(False, n, heads, kvh, 2000, 2000, 128, False).order == BY_CLASS
+    step = 256 // (heads // kvh)
+    tiles = [-(-2000 // step)] * n
+    order = tile_order([2000] * n, tiles, step)
+    even = sum(2000 - (tiles[s] - 1 - t) * step for s, t in order) * kvh / 256
+    assert rounds(order, [2000] * n, tiles, step, kvh) <= 1.25 * even
+    whole = sorted(order, key=lambda x: (x[0], -x[1]))
+    assert rounds(whole, [2000] * n, tiles, step, kvh) > 1.25 * even

@@ -481,7 +481,7 @@ static int paged_attention_impl(const vapi_kv_pool* pool, uint32_t layer, const 
   a.pf_min_q = 2;
   a.pf_seqs = listed ? pf->seqs : nullptr;
   a.pf_seqs_n = pf_n;
-  a.pf_sort = 0;
+  a.pf_order = kPfListOrder;
   a.kv_parts = FastDiv(1);
   a.g_real = a.group;
   a.hd = g.d;

@@ -71,7 +71,7 @@ struct AttnArgs {
   // batch - 1); the host names the sequences with prefill rows.
   const uint32_t* pf_seqs;
   uint32_t pf_seqs_n;
-  uint32_t pf_sort;  // prefill: items in descending order of work (prefill_sorts)
+  uint32_t pf_order;  // prefill: the order of the items (PfOrder)
   // decode: a group of G > 16 query heads per kv head runs as n = kv_parts
   // virtual kv heads of P = group = ceil(G / n) query heads each (kvh and
   // group then count the virtual ones; the last part of a group may hold
@@ -90,11 +90,14 @@ struct AttnArgs {
 // 8 XCDs (linear id % 8); each XCD here gets a contiguous range of work
 // items, so the q-tiles of one (sequence, kv head), which read the same K/V,
 // run at the same time under one L2.
+__device__ __forceinline__ uint32_t deal_remap(uint32_t lin, uint32_t n, uint32_t parts) {
+  const uint32_t x = lin % parts, i = lin / parts;
+  const uint32_t per = n / parts, extra = n % parts;  // part x gets per + (x < extra)
+  return x * per + min(x, extra) + i;
+}
 __device__ __forceinline__ uint32_t xcd_remap(uint32_t lin, uint32_t n) {
   constexpr uint32_t kXcds = 8;
-  const uint32_t x = lin % kXcds, i = lin / kXcds;
-  const uint32_t per = n / kXcds, extra = n % kXcds;  // XCD x gets per + (x < extra)
-  return x * per + min(x, extra) + i;
+  return deal_remap(lin, n, kXcds);
 }
 
 // A prefill work item: query tile qt of list entry li (sequence seq, its rows
@@ -103,6 +106,19 @@ struct PfItem {
   uint32_t li, seq, qt, kh, q0, len_q;
   int32_t len_k;
 };
+
+// The sum or maximum of x over the wave, in every lane.
+template <typename Op>
+__device__ __forceinline__ uint32_t wave_reduce(uint32_t x, Op op) {
+  x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xF, 0xF, false));  // row_ror:8
+  x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x124, 0xF, 0xF, false));  // row_ror:4
+  x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x122, 0xF, 0xF, false));  // row_ror:2
+  x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x121, 0xF, 0xF, false));  // row_ror:1
+  const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  x = op(r[0], r[1]);
+  const auto q = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  return op(q[0], q[1]);
+}
 
 // Item `i` of a prefill launch over a.pf_seqs_n list entries of at most
 // `qtiles` tiles of `rows` rows each; false when there is none (a sequence
@@ -118,7 +134,21 @@ struct PfItem {
 // fresh f16 prompts of 40-2,943 tokens (28 q / 4 kv heads) 404 -> 181 us
 // (the longest prompt's tiles had all run on one XCD), 16 chunks of 30-1,500
 // over ~500 earlier keys (32 q / 32 kv heads) 484 -> 295 us, config 3's
-// equal sequences 1,065 -> 1,057 us. Launches of one tile per sequence and
+// equal sequences 1,065 -> 1,057 us.
+// With one or two kv heads a sequence's tiles spread over 8 or 4 XCDs. In
+// launches of a few rounds, whole sequences one after the other then leave the
+// last one's long tiles to the end, where a sequence to an XCD had paired long
+// tiles with short ones: those walk the tiles by classes of work
+// (pf_tiles_to_class). Fresh prompts of 2,000 tokens, contiguous ranges /
+// whole sequences / classes: 4 (16 q / 2 kv heads) 101 / 115 / 83 us, 8 (8 q /
+// 1 kv head) 101 / 127 / 82. With more heads or rounds the classes part tiles
+// that share K/V and cost their search: 8 prompts (64 q / 8 kv heads) 623 us
+// whole, 648 by classes. Where all contexts are about equal and no tile is
+// short, every XCD takes a contiguous part of the walk, so that a sequence's
+// tiles share an L2 again: 8 chunks of 1,024 over 8,192 keys, contiguous ranges /
+// the walk dealt tile by tile / in parts: 32 q / 1 kv head 940 / 958 / 935 us,
+// head_dim 256 (8 q / 1 kv head) 570 / 592 / 563.
+// Launches of one tile per sequence and
 // of more sequences than lanes keep list order, which needs no walk over
 // the list (64 sequences of 32 fresh tokens: 16.8 us, 18.2 sorted; 17.4
 // before). So do launches of at most a workgroup per CU, where all items
@@ -133,9 +163,10 @@ __device__ __forceinline__ bool prefill_item(const AttnArgs& a, const uint32_t* 
                                              const uint32_t* __restrict__ cu_k, uint32_t i,
                                              uint32_t qtiles, uint32_t rows, uint32_t* tmp,
                                              PfItem& it) {
-  const uint32_t rank = i / a.kvh, n = a.pf_seqs_n;
+  uint32_t rank = i / a.kvh;
+  const uint32_t n = a.pf_seqs_n;
   it.kh = i - rank * a.kvh;
-  if (!a.pf_sort) {
+  if (a.pf_order == kPfListOrder) {
     it.li = rank / qtiles;
     it.qt = qtiles - 1 - (rank - it.li * qtiles);
     it.seq = a.pf_seqs ? a.pf_seqs[it.li] : it.li;
@@ -157,10 +188,45 @@ __device__ __forceinline__ bool prefill_item(const AttnArgs& a, const uint32_t* 
         nt = min((uint32_t)(((uint64_t)len_q * a.group + rows - 1) / rows), qtiles);
     }
   }
+  uint32_t first = 0, here = nt;  // this lane's tiles in earlier classes, in the rank's
+  const uint64_t some = __ballot(nt > 0);
+  if (some == 0) return false;
+  if (a.pf_order >= kPfParts) {
+    auto total = [&](uint32_t t) {
+      return (uint32_t)__builtin_amdgcn_readfirstlane(
+          wave_reduce(t, [](uint32_t x, uint32_t y) { return x + y; }));
+    };
+    // (With a left window, or without the causal mask, a sequence's tiles have
+    // equal work.)
+    const bool causal = a.wl < 0 && a.wr >= 0;
+    const uint32_t step = max(rows / a.group, 1u);
+    const uint32_t ref = __builtin_amdgcn_readlane(key, (uint32_t)__builtin_ctzll(some));
+    if (__all(nt == 0 || (key >= ref - ref / 8 && key <= ref + ref / 8 &&
+                          !(causal && pf_short_tile(ref, key, nt, step))))) {
+      const uint32_t tiles = total(nt);
+      if (rank < tiles) rank = deal_remap(rank, tiles, 8 / a.kvh);
+    } else if (a.pf_order == kPfByClass && causal) {
+      const uint32_t longest = __builtin_amdgcn_readfirstlane(
+          wave_reduce(nt ? key : 0u, [](uint32_t x, uint32_t y) { return max(x, y); }));
+      if (__any(pf_short_tile(longest, key, nt, step))) {
+        const float per_step = 1.f / (float)step;
+        uint32_t before = 0;                   // the launch's tiles in earlier classes
+        uint32_t lo = 0, hi = kPfClasses - 1;  // the first class whose end passes the rank
+        while (lo < hi) {
+          const uint32_t mid = (lo + hi) / 2;
+          const uint32_t t = pf_tiles_to_class(mid, longest, key, nt, per_step), sum = total(t);
+          if (rank < sum) hi = mid;
+          else lo = mid + 1, first = t, before = sum;
+        }
+        here = pf_tiles_to_class(lo, longest, key, nt, per_step) - first;
+        rank -= before;
+      }
+    }
+  }
   // Tiles of the sequences walked before this lane's.
   uint32_t start = 0;
   for (uint32_t s = wave; s < n; s += W) {
-    const uint32_t ks = __builtin_amdgcn_readlane(key, s), ns = __builtin_amdgcn_readlane(nt, s);
+    const uint32_t ks = __builtin_amdgcn_readlane(key, s), ns = __builtin_amdgcn_readlane(here, s);
     start += ks > key || (ks == key && s < lane) ? ns : 0u;
   }
   tmp[wave * 64 + lane] = start;
@@ -168,11 +234,11 @@ __device__ __forceinline__ bool prefill_item(const AttnArgs& a, const uint32_t* 
   start = 0;
 #pragma unroll
   for (int w = 0; w < W; ++w) start += tmp[w * 64 + lane];
-  const uint64_t hit = __ballot(rank >= start && rank - start < nt);
+  const uint64_t hit = __ballot(rank >= start && rank - start < here);
   if (hit == 0) return false;
   it.li = (uint32_t)__builtin_ctzll(hit);
   it.seq = __builtin_amdgcn_readlane(seq, it.li);
-  it.qt = __builtin_amdgcn_readlane(nt, it.li) - 1 -
+  it.qt = __builtin_amdgcn_readlane(nt - 1 - first, it.li) -
           (rank - __builtin_amdgcn_readlane(start, it.li));
   it.q0 = __builtin_amdgcn_readlane(q0, it.li);
   it.len_q = __builtin_amdgcn_readlane(len_q, it.li);

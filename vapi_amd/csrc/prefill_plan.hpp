@@ -26,11 +26,43 @@ VK_HD void key_range(int32_t p, int32_t len_k, int32_t wl, int32_t wr, int32_t& 
   hi = wr >= 0 ? pf_min(len_k - 1, p + wr) : len_k - 1;
 }
 
-// Launches whose items go in descending order of work (prefill_item says why).
+// How a launch's items are ordered (prefill_item says why).
 constexpr uint32_t kPfSortSeqs = 64;
 constexpr uint32_t kPfSortItems = 256;  // one per CU
-inline bool prefill_sorts(uint32_t n_seqs, uint32_t qtiles, uint64_t items) {
-  return n_seqs > 1 && n_seqs <= kPfSortSeqs && qtiles > 1 && items > kPfSortItems;
+constexpr uint32_t kPfFewHeads = 2;
+constexpr uint32_t kPfClassItems = 1024;
+enum PfOrder : uint32_t {
+  kPfListOrder,  // as the list has them
+  kPfSequences,  // sequences from the longest context to the shortest
+  kPfParts,      // the same; equal contexts in contiguous parts per XCD
+  kPfByClass,    // as kPfParts, or by classes of work
+};
+inline PfOrder prefill_order(uint32_t n_seqs, uint32_t kvh, uint32_t qtiles, uint64_t items,
+                             uint32_t n_split) {
+  const uint64_t wgs = items * n_split;
+  if (n_seqs <= 1 || n_seqs > kPfSortSeqs || qtiles <= 1 || wgs <= kPfSortItems)
+    return kPfListOrder;
+  if (kvh > kPfFewHeads || n_split > 1) return kPfSequences;
+  return items <= kPfClassItems ? kPfByClass : kPfParts;
+}
+
+// The order of a launch's tiles by classes of work (kPfByClass): classes, the
+// longest context over kPfClasses each, from the longest down; in a class the
+// sequences from the longest context down, each from its last tile to its first.
+// A tile has `step` keys less than the one after it. Returns the tiles of a
+// sequence of `key` keys and nt tiles in classes 0 .. c.
+constexpr uint32_t kPfClasses = 16;
+VK_HD uint32_t pf_tiles_to_class(uint32_t c, uint32_t longest, uint32_t key, uint32_t nt,
+                                 float per_step) {
+  if (c + 1 >= kPfClasses) return nt;
+  const uint32_t t = longest / kPfClasses * (kPfClasses - 1 - c);
+  if (key <= t) return 0;
+  return pf_min(nt, (uint32_t)((float)(key - t) * per_step) + 1);
+}
+// Whether a sequence's first tile has less than half of the longest's work: if
+// none has, the tiles are one class.
+VK_HD bool pf_short_tile(uint32_t longest, uint32_t key, uint32_t nt, uint32_t step) {
+  return nt > 0 && (uint64_t)(nt - 1) * step + longest / 2 > key;
 }
 
 // Bytes of one (item, split) partial block of a prefill key split: (m, l)
