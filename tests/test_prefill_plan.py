@@ -158,7 +158,7 @@ def rounds(order, lens_k, tiles, step, kvh, cus=32):
     return end
 
 
-@pytest.mark.parametrize("heads,kvh,n", [(16, 2, 4), (16, 2, 3), (8, 1, 8), (32, 1, 3)])
+@pytest.mark.parametrize("heads,kvh,n", [(16, 2, 4), (8, 1, 8), (32, 1, 3)])
 def test_equal_fresh_prompts_end_within_a_quarter_of_an_even_division(heads, kvh, n):
     """With one or two kv heads, where whole sequences one after the other
     ended up to half past it."""
