@@ -668,6 +668,8 @@ SPLIT_CASES = [
     (torch.float32, 16, 4, 64, 32, [100, 1], [3000, 2000], 500, "NHD"),
     (torch.float32, 32, 8, 128, 16, [512], [4096], None, "HND-bm"),
     (torch.float32, 16, 4, 80, 16, [100, 1], [3000, 2000], None, "HND"),
+    # 64 tiles in 4 shares each, most of them short.
+    (torch.bfloat16, 4, 1, 128, 16, [33] * 64, [6000] + [400] * 63, None, "HND"),
 ]
 
 
@@ -928,7 +930,11 @@ RANGE_CASES = [
     (torch.float16, 7, 1, 128, 32, [300, 301], [8000, 301], None, "NHD"),
     (torch.bfloat16, 8, 8, 64, 16, [520, 3, 256], [9100, 9100, 256], None, "HND"),
     (torch.bfloat16, 8, 4, 96, 16, [600, 90, 700], [7000, 6100, 6000], 4000, "HND"),
-    (torch.bfloat16, 4, 1, 128, 16, [33] * 64, [6000] + [400] * 63, None, "HND"),
+    # One sequence per lane of the plan.
+    (torch.bfloat16, 12, 3, 128, 16, [33] * 64, [6000] + [400] * 63, None, "HND"),
+    (torch.float32, 6, 3, 128, 16, [33] * 64, [3000] + [200] * 63, None, "HND"),
+    # Groups above 16: decode rows run in a launch of their own beside the ranges.
+    (torch.bfloat16, 34, 2, 128, 16, [700, 40, 300], [5000, 4000, 2500], None, "HND"),
     (torch.float32, 8, 4, 128, 16, [130, 70, 200], [4000, 900, 3100], None, "HND"),
     (torch.float32, 8, 2, 80, 16, [100, 150, 17], [3000, 3000, 2500], 1500, "NHD"),
     (torch.float32, 4, 2, 64, 32, [17] * 40, [2000] * 5 + [100] * 35, None, "HND"),
@@ -939,12 +945,21 @@ RANGE_CASES = [
                          ids=lambda c: f"{str(c[0])[6:]}-g{c[1] // c[2]}-d{c[3]}-n{len(c[5])}-w{c[7]}")
 def test_prefill_in_ranges_of_equal_work_matches_the_oracle(case):
     """Lengths whose tiles leave the GPU idle: ranges that end inside tiles,
-    cover several and span kv heads; with decode rows beside them too, and
-    against the same call unsplit (deterministic)."""
+    cover several and span kv heads, and against the same call unsplit
+    (deterministic). With a decode row in the batch too: beside ranges where
+    the decode has its own launch (f32, groups above 16), else in the mixed
+    launch, which has none."""
     dtype, heads, kvh, d, bs, lens_q, lens_k, window, layout = case
     rng = np.random.default_rng(zlib.crc32(str(case).encode()))
     left = None if window is None else window - 1
+    f32, kernel_d = dtype == torch.float32, 64 if d <= 64 else 128
+    ranges = 0
     for rows in (lens_q, [1] + lens_q[1:]):
+        n = sum(1 for x in rows if x > 1)
+        own_launch = n == len(rows) or f32 or heads // kvh > 16
+        r = route(f32, n, heads, kvh, max(rows), max(lens_k), kernel_d)
+        assert r.ranges or n < len(rows)
+        ranges += bool(r.ranges) and own_launch
         c, q, batch = random_case(rng, dtype, heads, kvh, d, bs, rows, lens_k, layout)
         want = oracle_out(q, c, 0, batch, d ** -0.5, window)
         tol = (1e-5 if dtype == torch.float32 else
@@ -955,6 +970,8 @@ def test_prefill_in_ranges_of_equal_work_matches_the_oracle(case):
             got = torch.full_like(q, float("nan"))
             paged_attention_prepared(q, c, 0, prep, d ** -0.5, left, out=got)
             assert max_abs(got, want) <= tol
+    # Decode rows beside ranges: the batches of 40 and 64, and the wide group.
+    assert ranges == (2 if heads // kvh > 16 or (f32 and len(lens_q) >= 40) else 1)
 
 
 @pytest.mark.parametrize("dtype,heads,kvh,n,q_len", [(torch.bfloat16, 32, 8, 15, 128),
