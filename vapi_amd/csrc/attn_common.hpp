@@ -89,7 +89,8 @@ struct AttnArgs {
 // Workgroup -> work item. The hardware deals workgroups round-robin to the
 // 8 XCDs (linear id % 8); each XCD here gets a contiguous range of work
 // items, so the q-tiles of one (sequence, kv head), which read the same K/V,
-// run at the same time under one L2.
+// run at the same time under one L2. (deal_remap: over `parts` XCDs, of items
+// dealt to them in turn.)
 __device__ __forceinline__ uint32_t deal_remap(uint32_t lin, uint32_t n, uint32_t parts) {
   const uint32_t x = lin % parts, i = lin / parts;
   const uint32_t per = n / parts, extra = n % parts;  // part x gets per + (x < extra)

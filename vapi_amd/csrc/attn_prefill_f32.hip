@@ -16,7 +16,7 @@
 // 3.0e-7, head_dim 80 with a window 3.9e-7 -> 3.0e-7, head_dim 96 fresh
 // 3.4e-7 -> 2.6e-7. Six bf16 MFMAs at 1/16 of an f32 MFMA's cost: 2.7 times
 // the f32 rate. 8 chunks of 512 over 4,096 keys (32 q / 8 kv heads) 2,478 ->
-// 1,148 us (105 -> 225 TFLOP/s), the 4 ragged chunks 442 -> 192 us.
+// 1,165 us (105 -> 221 TFLOP/s), the 4 ragged chunks 442 -> 193 us.
 //
 // Values whose h would not be finite (infinities, NaN, |x| above the largest
 // bf16) have no such split: their l is NaN, which reaches every sum that the
