@@ -12,19 +12,29 @@ extern "C" {
 // out: items, query tiles, n_split, ranges, workspace bytes of the ranges,
 // the items' order (PfOrder).
 void plan_route16(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_q, uint32_t max_k,
-                  uint32_t head_dim, int split_ok, uint64_t ws_bytes, uint64_t* out) {
+                  uint32_t head_dim, uint32_t row_bytes, int split_ok, uint64_t ws_bytes,
+                  uint64_t* out) {
   const PfRoute r = pf_route(n_seqs, kvh, group, max_q, max_k, head_dim, split_ok, ws_bytes);
   out[0] = r.items, out[1] = r.qtiles, out[2] = r.n_split, out[3] = r.ranges.ranges;
   out[4] = r.ranges.bytes;
-  out[5] = prefill_order(n_seqs, kvh, r.qtiles, r.items, r.n_split);
+  out[5] = prefill_order(n_seqs, kvh, r.qtiles, r.items, r.n_split, max_k, row_bytes,
+                         pf_slots(head_dim));
 }
 
 void plan_route_f32(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_q, uint32_t max_k,
-                    uint32_t head_dim, int split_ok, uint64_t ws_bytes, uint64_t* out) {
+                    uint32_t head_dim, uint32_t row_bytes, int split_ok, uint64_t ws_bytes,
+                    uint64_t* out) {
   const F32Route r = f32_route(n_seqs, kvh, group, max_q, max_k, head_dim, split_ok, ws_bytes);
   out[0] = r.plan.items, out[1] = r.plan.qtiles, out[2] = r.n_split, out[3] = r.ranges.ranges;
   out[4] = r.ranges.bytes;
-  out[5] = prefill_order(n_seqs, kvh, r.plan.qtiles, r.plan.items, r.n_split);
+  out[5] = prefill_order(n_seqs, kvh, r.plan.qtiles, r.plan.items, r.n_split, max_k, row_bytes,
+                         256);
+}
+
+// (list entry, kv head, tile) of every item of a launch in kPfListParts.
+void plan_list_parts(uint32_t n_seqs, uint32_t kvh, uint32_t qtiles, uint32_t* out) {
+  for (uint32_t i = 0; i < n_seqs * kvh * qtiles; ++i)
+    pf_list_part(i, n_seqs, kvh, qtiles, out[3 * i], out[3 * i + 1], out[3 * i + 2]);
 }
 
 }  // extern "C"

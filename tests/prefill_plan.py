@@ -7,7 +7,7 @@ from functools import lru_cache
 from pathlib import Path
 
 ANY_BYTES = (1 << 64) - 1
-LIST_ORDER, SEQUENCES, PARTS, BY_CLASS = range(4)  # PfOrder
+LIST_ORDER, LIST_PARTS, SEQUENCES, PARTS, BY_CLASS = range(5)  # PfOrder
 
 
 @lru_cache(maxsize=None)
@@ -32,14 +32,15 @@ class Route:
     rows: int
 
 
-def route(f32, n_seqs, heads, kvh, max_q, max_k, head_dim, split_ok=True, ws_bytes=ANY_BYTES):
+def route(f32, n_seqs, heads, kvh, max_q, max_k, head_dim, split_ok=True, ws_bytes=ANY_BYTES,
+          pool_dim=None):
     """How a prefill launch over n_seqs listed sequences runs. `head_dim`: the
-    kernel's (64, 128 or 256)."""
+    kernel's (64, 128 or 256); `pool_dim`: the pool's, where it is another."""
     out = (ctypes.c_uint64 * 6)()
     fn = _lib().plan_route_f32 if f32 else _lib().plan_route16
     u32 = ctypes.c_uint32
     fn(u32(n_seqs), u32(kvh), u32(heads // kvh), u32(max_q), u32(max_k), u32(head_dim),
-       int(split_ok), ctypes.c_uint64(ws_bytes), out)
+       u32((pool_dim or head_dim) * (4 if f32 else 2)), int(split_ok), ctypes.c_uint64(ws_bytes), out)
     rows = 128 if f32 or head_dim == 256 else 256
     return Route(out[0], out[1], out[2], out[3], out[4], out[5], rows)
 
@@ -63,3 +64,11 @@ def tile_order(lens_k, tiles, step):
                             (ctypes.c_uint32 * n)(*tiles), ctypes.c_uint32(step), out)
     assert bad == 0, bad
     return [(out[2 * i], out[2 * i + 1]) for i in range(total)]
+
+
+def item_order(n_seqs, qtiles, kvh):
+    """The (list entry, kv head, tile) of every item of a launch in LIST_PARTS."""
+    out = (ctypes.c_uint32 * (3 * n_seqs * qtiles * kvh))()
+    _lib().plan_list_parts(ctypes.c_uint32(n_seqs), ctypes.c_uint32(kvh), ctypes.c_uint32(qtiles),
+                           out)
+    return [tuple(out[3 * i:3 * i + 3]) for i in range(n_seqs * qtiles * kvh)]

@@ -16,7 +16,7 @@ import pytest
 import torch
 
 import oracle
-from prefill_plan import BY_CLASS, LIST_ORDER, PARTS, SEQUENCES, route
+from prefill_plan import BY_CLASS, LIST_ORDER, LIST_PARTS, PARTS, SEQUENCES, route
 from vapi_amd import _lib, workload
 from vapi_amd.attention import (ForwardBatch, PreparedAttention, paged_attention,
                                 paged_attention_prepared, paged_attention_windowed)
@@ -760,6 +760,50 @@ def test_every_tile_of_a_ragged_prefill_batch_is_computed_once(case):
                                             deterministic=f32)  # (no ranges)
         if not decode_rows:
             assert route(f32, n, heads, kvh, max(lens_q), max(lens_k), d, not f32).order == order
+        want = oracle_out(q, c, 0, batch, d ** -0.5)
+        got = torch.full_like(q, float("nan"))
+        paged_attention_prepared(q, c, 0, prep, d ** -0.5, out=got)
+        tol = (1e-5 if f32 else
+               (2e-2 if dtype == torch.bfloat16 else 1e-2) * float(want.abs().max()))
+        assert max_abs(got, want) <= tol
+
+
+SHORT_CASES = [
+    # dtype, heads, kvh, d, n_seqs, most queries each, keys before them, the order
+    (torch.bfloat16, 16, 16, 80, 20, 40, 0, LIST_PARTS),     # one tile each, few keys
+    (torch.float16, 24, 3, 64, 70, 30, 300, LIST_PARTS),     # at most a workgroup per slot
+    (torch.bfloat16, 28, 4, 96, 64, 60, 0, LIST_PARTS),      # two tiles each, fewer keys
+    (torch.bfloat16, 21, 3, 64, 90, 50, 0, LIST_PARTS),      # the same, past 64 sequences
+    (torch.float16, 24, 24, 96, 13, 200, 300, SEQUENCES),    # one tile each, sorted
+    (torch.bfloat16, 12, 12, 128, 64, 20, 200, SEQUENCES),
+    (torch.float32, 16, 16, 80, 20, 128, 300, SEQUENCES),
+    (torch.bfloat16, 32, 32, 80, 70, 8, 200, LIST_ORDER),    # past the sort
+    (torch.bfloat16, 32, 32, 64, 65, 8, 0, LIST_ORDER),      # past four rounds
+    (torch.bfloat16, 32, 32, 80, 40, 8, 0, LIST_PARTS),      # rows that share lines
+]
+
+
+@pytest.mark.parametrize("case", SHORT_CASES,
+                         ids=lambda c: f"{str(c[0])[6:]}-kvh{c[2]}-d{c[3]}-n{c[4]}-k{c[6]}")
+def test_prefill_batches_of_short_sequences_are_computed_once(case):
+    """One tile per sequence, or a few short ones: the orders of those launches,
+    alone and with decode rows beside them."""
+    dtype, heads, kvh, d, n, top, before, order = case
+    rng = np.random.default_rng(zlib.crc32(str(case).encode()))
+    f32 = dtype == torch.float32
+    lens_q = [int(x) for x in rng.integers(2, top + 1, n)]
+    lens_q[n // 3] = top
+    lens_k = [l + int(x) for l, x in zip(lens_q, rng.integers(0, 2 * before + 1, n))]
+    kernel_d = 64 if d <= 64 else 128
+    for decode_rows in (False, True):
+        if decode_rows:
+            lens_q[n // 2] = 1
+        c, q, batch = random_case(rng, dtype, heads, kvh, d, 16, lens_q, lens_k, "HND")
+        prep = PreparedAttention.from_batch(batch, DEV, cache=c, num_heads=heads,
+                                            deterministic=True)  # (whole tiles)
+        if not decode_rows:
+            assert route(f32, n, heads, kvh, max(lens_q), max(lens_k), kernel_d, False,
+                         pool_dim=d).order == order
         want = oracle_out(q, c, 0, batch, d ** -0.5)
         got = torch.full_like(q, float("nan"))
         paged_attention_prepared(q, c, 0, prep, d ** -0.5, out=got)

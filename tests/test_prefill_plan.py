@@ -6,7 +6,8 @@ import heapq
 import numpy as np
 import pytest
 
-from prefill_plan import BY_CLASS, check_walk, route, tile_order
+from prefill_plan import (BY_CLASS, LIST_ORDER, LIST_PARTS, SEQUENCES, check_walk, item_order, route,
+                          tile_order)
 
 
 def equal(f32, n, heads, kvh, q, k, d=128):
@@ -170,3 +171,43 @@ def test_equal_fresh_prompts_end_within_a_quarter_of_an_even_division(heads, kvh
     assert rounds(order, [2000] * n, tiles, step, kvh) <= 1.25 * even
     whole = sorted(order, key=lambda x: (x[0], -x[1]))
     assert rounds(whole, [2000] * n, tiles, step, kvh) > 1.25 * even
+
+
+@pytest.mark.parametrize("heads,kvh,n", [(16, 16, 40), (24, 12, 40), (8, 8, 64)])
+def test_ragged_sequences_of_one_tile_each_do_not_end_on_a_long_one(heads, kvh, n):
+    """A round or more of items: the launch ends within a sixth of the longest
+    item past an even division, where the list dealt as it is ends a fifth or more
+    of one past it."""
+    rng = np.random.default_rng(4)
+    lens = [int(x) for x in np.clip(np.exp(rng.normal(np.log(300), 0.75, n)), 33, 4000)]
+    lens[-1] = max(lens) + 1
+    r = route(False, n, heads, kvh, 20, max(lens), 128, False)
+    assert r.qtiles == 1 and r.order == SEQUENCES
+    walk = sorted(range(n), key=lambda i: -lens[i])
+    even = max(sum(lens) * kvh / 256, max(lens))
+    assert rounds([(s, 0) for s in walk], lens, [1] * n, 1, kvh) <= even + max(lens) / 6
+    assert rounds([(s, 0) for s in range(n)], lens, [1] * n, 1, kvh) > even + max(lens) / 5
+
+
+def test_short_sequences_keep_list_order():
+    """Where the sort costs more than it gives (few keys, all items at once, or
+    many rounds of them), and a sequence's tiles stay on one XCD."""
+    for n, heads, kvh, q, k, d, want in ((64, 16, 16, 32, 32, 128, LIST_PARTS),
+                                         (64, 32, 8, 12, 600, 64, LIST_PARTS),
+                                         (64, 32, 32, 12, 600, 128, LIST_ORDER),
+                                         (64, 16, 16, 12, 600, 128, LIST_ORDER),
+                                         (130, 32, 32, 50, 50, 128, LIST_ORDER),
+                                         (130, 32, 32, 50, 50, 80, LIST_PARTS),
+                                         (64, 28, 4, 64, 64, 128, LIST_PARTS),
+                                         (130, 28, 4, 50, 50, 64, LIST_PARTS),
+                                         (40, 28, 4, 128, 128, 128, SEQUENCES)):
+        kernel_d = 64 if d <= 64 else 128
+        assert route(False, n, heads, kvh, q, k, kernel_d, False, pool_dim=d).order == want
+    for n, qtiles, kvh in ((64, 2, 4), (130, 2, 4), (20, 1, 16), (3, 5, 3)):
+        items = item_order(n, qtiles, kvh)
+        assert sorted(items) == [(s, h, t) for s in range(n) for h in range(kvh)
+                                 for t in range(qtiles)]
+        xcds = [{(i, s) for i, (s, h, t) in enumerate(items) if i % 8 == x} for x in range(8)]
+        # A sequence on two XCDs at most, where each holds a sequence or more.
+        if n >= 8:
+            assert max(sum(any(s == q for _, q in x) for x in xcds) for s in range(n)) <= 2

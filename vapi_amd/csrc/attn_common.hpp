@@ -86,21 +86,6 @@ struct AttnArgs {
   uint32_t hd;
 };
 
-// Workgroup -> work item. The hardware deals workgroups round-robin to the
-// 8 XCDs (linear id % 8); each XCD here gets a contiguous range of work
-// items, so the q-tiles of one (sequence, kv head), which read the same K/V,
-// run at the same time under one L2. (deal_remap: over `parts` XCDs, of items
-// dealt to them in turn.)
-__device__ __forceinline__ uint32_t deal_remap(uint32_t lin, uint32_t n, uint32_t parts) {
-  const uint32_t x = lin % parts, i = lin / parts;
-  const uint32_t per = n / parts, extra = n % parts;  // part x gets per + (x < extra)
-  return x * per + min(x, extra) + i;
-}
-__device__ __forceinline__ uint32_t xcd_remap(uint32_t lin, uint32_t n) {
-  constexpr uint32_t kXcds = 8;
-  return deal_remap(lin, n, kXcds);
-}
-
 // A prefill work item: query tile qt of list entry li (sequence seq, its rows
 // q0 .. q0 + len_q - 1 and context len_k), kv head kh.
 struct PfItem {
@@ -149,13 +134,27 @@ __device__ __forceinline__ uint32_t wave_reduce(uint32_t x, Op op) {
 // tiles share an L2 again: 8 chunks of 1,024 over 8,192 keys, contiguous ranges /
 // the walk dealt tile by tile / in parts: 32 q / 1 kv head 940 / 958 / 935 us,
 // head_dim 256 (8 q / 1 kv head) 570 / 592 / 563.
-// Launches of one tile per sequence and
-// of more sequences than lanes keep list order, which needs no walk over
-// the list (64 sequences of 32 fresh tokens: 16.8 us, 18.2 sorted; 17.4
-// before). So do launches of at most a workgroup per CU, where all items
-// start at once and their order changes nothing: 6 x 100-200 fresh tokens
-// at head_dim 64 (96 items) take 10.8 us, 11.3 sorted, 3 x 100-200 of 28 q /
-// 4 kv heads at head_dim 96 12.2, 12.5 sorted.
+// Launches of more sequences than lanes keep list order, which needs no walk
+// over the list (~1.3 us per workgroup). So do launches of several tiles per
+// sequence and at most a workgroup per CU, where all items start at once: 6 x
+// 100-200 fresh tokens at head_dim 64 (96 items) take 10.8 us, 11.3 sorted.
+// With one tile per sequence (bf16; list order / contiguous parts of the list
+// per XCD / sorted, us) the walk pays from a round of items to three, where the
+// longest is long beside it: 40 x 10-60 tokens over ~300 keys (16 q / 16 kv
+// heads) 54.3 / 46.8 / 43.8, 20 x 10-180 fresh 18.7 / 22.2 / 16.8; equal
+// contexts lose it (60 x 60 over 900, 24 q / 12 kv heads: 124.2 / - / 126.3).
+// Contiguous parts, where a sequence's heads stay together, where all items
+// start at once (64 x 4-12 over ~200, 32 q / 8 kv heads at head_dim 64: 31.6 /
+// 28.3 / 29.9) or are short (64 x 32 fresh, 16 q / 16 kv heads: 22.0 / 21.4 /
+// 24.9). Past a few rounds the dealt list balances itself: 64 x 4-12 over ~200
+// (32 q / 32 kv heads) 92.5 / 109.5 / 100.0, 130 x 10-50 fresh 91.3 / 95.6 / -;
+// short ones stay in parts there too where a head's rows share L2 lines with
+// its neighbours' (the same 130 at head_dim 80: 91.7 / 87.5).
+// Several tiles of a few keys each cost less than the walk (and in list order
+// a sequence's tiles part where the kv heads are fewer than the XCDs): 64 x
+// 4-64 fresh, 28 q / 4 kv heads at head_dim 80, parts / sorted 16.9 / 20.5. Up
+// to 128 keys the walk wins again where lengths differ (40 x 8-128: 26.4 / 21.6)
+// and loses where they do not (40 x 128: 29.7 / 33.7).
 // Each of the workgroup's W waves holds one sequence per lane and counts the
 // tiles before it among its share of the others; `tmp` (W x 64 words of LDS)
 // adds the shares up. Every thread of the workgroup calls this.
@@ -164,12 +163,16 @@ __device__ __forceinline__ bool prefill_item(const AttnArgs& a, const uint32_t* 
                                              const uint32_t* __restrict__ cu_k, uint32_t i,
                                              uint32_t qtiles, uint32_t rows, uint32_t* tmp,
                                              PfItem& it) {
-  uint32_t rank = i / a.kvh;
   const uint32_t n = a.pf_seqs_n;
+  uint32_t rank = i / a.kvh;
   it.kh = i - rank * a.kvh;
-  if (a.pf_order == kPfListOrder) {
-    it.li = rank / qtiles;
-    it.qt = qtiles - 1 - (rank - it.li * qtiles);
+  if (a.pf_order <= kPfListParts) {
+    if (a.pf_order == kPfListParts) {
+      pf_list_part(i, n, a.kvh, qtiles, it.li, it.kh, it.qt);
+    } else {
+      it.li = rank / qtiles;
+      it.qt = qtiles - 1 - (rank - it.li * qtiles);
+    }
     it.seq = a.pf_seqs ? a.pf_seqs[it.li] : it.li;
     if (it.seq >= a.batch) return false;
     it.q0 = cu_q[it.seq];

@@ -27,23 +27,72 @@ VK_HD void key_range(int32_t p, int32_t len_k, int32_t wl, int32_t wr, int32_t& 
 }
 
 // How a launch's items are ordered (prefill_item says why).
+constexpr uint32_t kLine = 128;  // bytes of an L2 line
 constexpr uint32_t kPfSortSeqs = 64;
 constexpr uint32_t kPfSortItems = 256;  // one per CU
 constexpr uint32_t kPfFewHeads = 2;
 constexpr uint32_t kPfClassItems = 1024;
+constexpr uint32_t kPfSortRounds = 3;
+constexpr uint32_t kPfPartsRounds = 4;
+constexpr uint32_t kPfShortKeys = 128;
+constexpr uint32_t kPfShortTileKeys = 64;
 enum PfOrder : uint32_t {
   kPfListOrder,  // as the list has them
+  kPfListParts,  // the same, in contiguous parts per XCD
   kPfSequences,  // sequences from the longest context to the shortest
   kPfParts,      // the same; equal contexts in contiguous parts per XCD
   kPfByClass,    // as kPfParts, or by classes of work
 };
+// `keys`: the most that an item walks; `row`: bytes of a head's row; `slots`:
+// workgroups the GPU runs at once.
 inline PfOrder prefill_order(uint32_t n_seqs, uint32_t kvh, uint32_t qtiles, uint64_t items,
-                             uint32_t n_split) {
+                             uint32_t n_split, uint64_t keys, uint32_t row, uint32_t slots) {
   const uint64_t wgs = items * n_split;
-  if (n_seqs <= 1 || n_seqs > kPfSortSeqs || qtiles <= 1 || wgs <= kPfSortItems)
-    return kPfListOrder;
+  if (n_seqs <= 1) return kPfListOrder;
+  if (qtiles <= 1) {
+    if (n_split > 1) return kPfListOrder;
+    if (wgs <= slots) return kPfListParts;
+    if (keys <= kPfShortKeys)
+      return row % kLine || wgs <= kPfPartsRounds * (uint64_t)slots ? kPfListParts : kPfListOrder;
+    return n_seqs <= kPfSortSeqs && wgs <= kPfSortRounds * (uint64_t)slots ? kPfSequences
+                                                                           : kPfListOrder;
+  }
+  if (keys <= kPfShortTileKeys && n_split == 1) return kPfListParts;
+  if (n_seqs > kPfSortSeqs || wgs <= kPfSortItems) return kPfListOrder;
   if (kvh > kPfFewHeads || n_split > 1) return kPfSequences;
   return items <= kPfClassItems ? kPfByClass : kPfParts;
+}
+
+// Workgroup -> work item. The hardware deals workgroups round-robin to the
+// 8 XCDs (linear id % 8); each XCD here gets a contiguous range of work
+// items, so the q-tiles of one (sequence, kv head), which read the same K/V,
+// run at the same time under one L2. (deal_remap: over `parts` XCDs, of items
+// dealt to them in turn.)
+VK_HD uint32_t deal_remap(uint32_t lin, uint32_t n, uint32_t parts) {
+  const uint32_t x = lin % parts, i = lin / parts;
+  const uint32_t per = n / parts, extra = n % parts;  // part x gets per + (x < extra)
+  return x * per + pf_min(x, extra) + i;
+}
+VK_HD uint32_t xcd_remap(uint32_t lin, uint32_t n) {
+  constexpr uint32_t kXcds = 8;
+  return deal_remap(lin, n, kXcds);
+}
+
+// Item i of a launch in kPfListParts: tile fastest, then kv head, then list
+// entry li.
+VK_HD void pf_list_part(uint32_t i, uint32_t n_seqs, uint32_t kvh, uint32_t qtiles, uint32_t& li,
+                        uint32_t& kh, uint32_t& qt) {
+  i = xcd_remap(i, n_seqs * qtiles * kvh);
+  const uint32_t head = i / qtiles;
+  qt = qtiles - 1 - (i - head * qtiles);
+  li = head / kvh;
+  kh = head - li * kvh;
+}
+
+// The most keys that an item walks, with at most max_q queries and max_k keys
+// per sequence and the left window wl.
+inline uint64_t prefill_keys(uint32_t max_q, uint32_t max_k, int32_t wl) {
+  return wl >= 0 ? std::min<uint64_t>(max_k, (uint64_t)wl + max_q) : max_k;
 }
 
 // The order of a launch's tiles by classes of work (kPfByClass): classes, the
