@@ -18,7 +18,7 @@ void plan_route16(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_q,
   out[0] = r.items, out[1] = r.qtiles, out[2] = r.n_split, out[3] = r.ranges.ranges;
   out[4] = r.ranges.bytes;
   out[5] = prefill_order(n_seqs, kvh, r.qtiles, r.items, r.n_split, max_k, row_bytes,
-                         pf_slots(head_dim));
+                         pf_slots(head_dim), false);
 }
 
 void plan_route_f32(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_q, uint32_t max_k,
@@ -28,7 +28,7 @@ void plan_route_f32(uint32_t n_seqs, uint32_t kvh, uint32_t group, uint32_t max_
   out[0] = r.plan.items, out[1] = r.plan.qtiles, out[2] = r.n_split, out[3] = r.ranges.ranges;
   out[4] = r.ranges.bytes;
   out[5] = prefill_order(n_seqs, kvh, r.plan.qtiles, r.plan.items, r.n_split, max_k, row_bytes,
-                         256);
+                         256, true);
 }
 
 // (list entry, kv head, tile) of every item of a launch in kPfListParts.

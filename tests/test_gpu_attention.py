@@ -776,7 +776,8 @@ SHORT_CASES = [
     (torch.bfloat16, 21, 3, 64, 90, 50, 0, LIST_PARTS),      # the same, past 64 sequences
     (torch.float16, 24, 24, 96, 13, 200, 300, SEQUENCES),    # one tile each, sorted
     (torch.bfloat16, 12, 12, 128, 64, 20, 200, SEQUENCES),
-    (torch.float32, 16, 16, 80, 20, 128, 300, SEQUENCES),
+    (torch.float32, 16, 16, 80, 20, 128, 300, LIST_ORDER),   # f32: as listed
+    (torch.float32, 16, 4, 64, 40, 63, 0, SEQUENCES),        # or walked
     (torch.bfloat16, 32, 32, 80, 70, 8, 200, LIST_ORDER),    # past the sort
     (torch.bfloat16, 32, 32, 64, 65, 8, 0, LIST_ORDER),      # past four rounds
     (torch.bfloat16, 32, 32, 80, 40, 8, 0, LIST_PARTS),      # rows that share lines

@@ -203,6 +203,9 @@ def test_short_sequences_keep_list_order():
                                          (40, 28, 4, 128, 128, 128, SEQUENCES)):
         kernel_d = 64 if d <= 64 else 128
         assert route(False, n, heads, kvh, q, k, kernel_d, False, pool_dim=d).order == want
+    # f32: as listed with one tile, walked with several.
+    assert route(True, 40, 16, 8, 128, 128, 64, False).order == LIST_ORDER
+    assert route(True, 10, 64, 8, 63, 63, 128, False).order == SEQUENCES
     for n, qtiles, kvh in ((64, 2, 4), (130, 2, 4), (20, 1, 16), (3, 5, 3)):
         items = item_order(n, qtiles, kvh)
         assert sorted(items) == [(s, h, t) for s in range(n) for h in range(kvh)

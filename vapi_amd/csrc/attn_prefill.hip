@@ -631,7 +631,8 @@ void launch_mixed(const AttnArgs& a_in, void* workspace, uint32_t max_q, uint32_
       --n_split;
   }
   c.pf_order = prefill_order(c.pf_seqs_n, c.kvh, qtiles, base, n_split,
-                             prefill_keys(max_q, max_k, c.wl), c.hd * sizeof(uint16_t), nwg);
+                             prefill_keys(max_q, max_k, c.wl), c.hd * sizeof(uint16_t), nwg,
+                             false);
   float* part = n_split > 1 ? (float*)split_ws : nullptr;
   const dim3 grid((uint32_t)(nwg + base * n_split)), block(256);
   // The decode's plan, or the prefill's order: one or the other per workgroup.
@@ -708,7 +709,7 @@ void launch_prefill(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, uint32
   const PfRangePlan rp = route.ranges;
   a.pf_order = prefill_order(a.pf_seqs_n, a.kvh, qtiles, base, n_split,
                              prefill_keys(max_q, max_k, a.wl), a.hd * sizeof(uint16_t),
-                             pf_slots(head_dim));
+                             pf_slots(head_dim), false);
   float* part = n_split > 1 ? (float*)split_ws : nullptr;
   const dim3 grid((uint32_t)(base * n_split)), block(kPfThreads);
 #define VK_PF(T, DD, PAD, DL)                                                                    \

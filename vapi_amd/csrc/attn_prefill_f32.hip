@@ -657,7 +657,8 @@ void launch_prefill_f32(const AttnArgs& a_in, uint32_t max_q, uint32_t max_k, ui
   const uint32_t qtiles = p.qtiles, n_split = route.n_split;
   const uint64_t items = p.items * n_split;
   a.pf_order = prefill_order(a.pf_seqs_n, a.kvh, qtiles, p.items, n_split,
-                             prefill_keys(max_q, max_k, a.wl), a.hd * sizeof(float), 256);
+                             prefill_keys(max_q, max_k, a.wl), a.hd * sizeof(float), 256,
+                             true);
   const uint32_t wgs = (uint32_t)((items + kPfF32Waves - 1) / kPfF32Waves);
   float* part = n_split > 1 ? (float*)split_ws : nullptr;
 #define VK_X3(DD, RT, SPLIT, PAD, CL)                                                            \

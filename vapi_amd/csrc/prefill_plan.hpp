@@ -44,20 +44,25 @@ enum PfOrder : uint32_t {
   kPfByClass,    // as kPfParts, or by classes of work
 };
 // `keys`: the most that an item walks; `row`: bytes of a head's row; `slots`:
-// workgroups the GPU runs at once.
+// workgroups the GPU runs at once. f32 launches keep the list's order with one
+// tile per sequence and walk several: their steps take 2.5 times as long, and
+// parts of the list end later (10 fresh sequences of 9-63 tokens, 64 q / 8 kv
+// heads: 15.9 us walked, 23.7 in parts; 40 of 8-128, 16 q / 8 kv heads: 33.9 as
+// listed, 38.5 in parts).
 inline PfOrder prefill_order(uint32_t n_seqs, uint32_t kvh, uint32_t qtiles, uint64_t items,
-                             uint32_t n_split, uint64_t keys, uint32_t row, uint32_t slots) {
+                             uint32_t n_split, uint64_t keys, uint32_t row, uint32_t slots,
+                             bool f32) {
   const uint64_t wgs = items * n_split;
   if (n_seqs <= 1) return kPfListOrder;
   if (qtiles <= 1) {
-    if (n_split > 1) return kPfListOrder;
+    if (n_split > 1 || f32) return kPfListOrder;
     if (wgs <= slots) return kPfListParts;
     if (keys <= kPfShortKeys)
       return row % kLine || wgs <= kPfPartsRounds * (uint64_t)slots ? kPfListParts : kPfListOrder;
     return n_seqs <= kPfSortSeqs && wgs <= kPfSortRounds * (uint64_t)slots ? kPfSequences
                                                                            : kPfListOrder;
   }
-  if (keys <= kPfShortTileKeys && n_split == 1) return kPfListParts;
+  if (keys <= kPfShortTileKeys && n_split == 1 && !f32) return kPfListParts;
   if (n_seqs > kPfSortSeqs || wgs <= kPfSortItems) return kPfListOrder;
   if (kvh > kPfFewHeads || n_split > 1) return kPfSequences;
   return items <= kPfClassItems ? kPfByClass : kPfParts;
