@@ -101,6 +101,15 @@ def test_a_small_workspace_does_not_run_a_launch_on_fewer_cus():
     assert route(True, 5, 16, 8, 512, 4096, 128, True, MIB16).ranges == 0
 
 
+def test_f32_batches_of_few_rows_get_the_ranges_their_workspace_is_for():
+    """Where the split kernel runs as ranges but not as tiles: the workspace asked
+    for holds them all."""
+    for n, heads, kvh, q, k in ((40, 8, 4, 59, 862), (40, 16, 8, 59, 862), (33, 8, 4, 40, 2000)):
+        r = route(True, n, heads, kvh, q, k, 128)
+        assert r.ranges == 256
+        assert route(True, n, heads, kvh, q, k, 128, True, r.range_bytes).ranges == 256
+
+
 def test_ranges_of_a_small_workspace_beat_its_tiles_or_shares():
     """A range's steps are at most those of the rounds of tiles or shares that
     the same workspace allows, all sequences as long as the longest."""

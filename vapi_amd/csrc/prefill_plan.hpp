@@ -426,6 +426,11 @@ inline F32Plan f32_range_plan(uint32_t n_seqs, uint32_t kvh, uint32_t group, uin
   // (Ranges balance the items that few rows would leave half idle: 40
   // sequences, 8 kv heads, 64 rows over ~1,000 keys: 378 us with f32 MFMAs.)
   p.x3 = p.x3 || all > 32;
+  // Its items fill the GPU one per CU, whatever kernel the tiles would take: with
+  // f32_plan's 1,024 here, ranges were priced against shares that nothing ran
+  // and the workspace asked for held none (40 chunks of 10-60 over ~300 keys, 8 q
+  // / 4 kv heads at head_dim 80: 81.7 us in f32 MFMAs, 44.3 in ranges).
+  if (p.x3) p.target = 256;
   p.row_tiles = 1;
   p.rows = x3_rows(1);
   p.qtiles = (uint32_t)((all + p.rows - 1) / p.rows);
